@@ -29,6 +29,7 @@
 #include <type_traits>
 
 #include <atomic>
+#include <cstring>
 #include <stdexcept>
 
 #include "device_math.h"
@@ -90,9 +91,10 @@ __device__ __forceinline__ uint4 gate_vec(uint4 v, const float* g) {
                     gate_pair(v.w, b.z, b.w));
 }
 
-template <typename T, int BM, int BN, int WM, int WN, typename RowPtr>
-__device__ __forceinline__ void finish_tile(const ConvParams& p, const floatx4 (&acc)[BM / (WM * 16)][BN / (WN * 16)],
-                                            RowPtr row_ptr, int m0, int n0, int M, int n_tiles);
+template <typename T, int BM, int BN, int WM, int WN, int BC = 16, typename RowPtr>
+__device__ __forceinline__ void finish_tile(const ConvParams& p,
+                                            const floatx4 (&acc)[BM * BC / (WM * 256)][BN / (WN * BC)], RowPtr row_ptr,
+                                            int m0, int n0, int M, int n_tiles, const float4* bias_pre);
 
 // PW: 1x1 convolution with stride 1 and no padding, where an output pixel
 // reads exactly its own input pixel and A rows are plain strided rows.
@@ -396,34 +398,39 @@ template <typename T, int BM, int BN, typename RowPtr>
 __device__ __forceinline__ void finish_staged(const ConvParams& p, RowPtr row_ptr, int m0, int n0, int M,
                                               int n_tiles, const float4* bias_pre);
 
+// Accumulators reach the epilogues as floatx4 groups acc[i][j] of four rows
+// by BC columns per 256 / (4 BC) lane groups: element e of lane l is row
+// i * 256 / BC + 4 (l / BC) + e, column j * BC + l % BC of the wave's tile.
+// BC = 16 is the 16x16 MFMA's layout (a group per block), BC = 32 the
+// 32x32 MFMA's (four groups per block, eight rows apart).
+
 // Stages the fp32 accumulator tile in LDS as [m][n] (row_ptr(r): LDS
 // address of staged row r, BN + 4 floats) and finishes it: with split K
 // (p.splits > 1) the tile goes to this split's plane of the workspace as is,
 // otherwise through the epilogue.  Caller has passed a barrier after its
 // last read of the LDS operand buffers.  bias_pre: null, or the bias of this
 // thread's staged-epilogue columns (staged_col) loaded ahead.
-template <typename T, int BM, int BN, int WM, int WN, typename RowPtr>
-__device__ __forceinline__ void finish_tile(const ConvParams& p, const floatx4 (&acc)[BM / (WM * 16)][BN / (WN * 16)],
-                                            RowPtr row_ptr, int m0, int n0, int M, int n_tiles,
-                                            const float4* bias_pre) {
-  constexpr int TM = BM / (WM * 16);
-  constexpr int TN = BN / (WN * 16);
+template <typename T, int BM, int BN, int WM, int WN, int BC, typename RowPtr>
+__device__ __forceinline__ void finish_tile(const ConvParams& p,
+                                            const floatx4 (&acc)[BM * BC / (WM * 256)][BN / (WN * BC)], RowPtr row_ptr,
+                                            int m0, int n0, int M, int n_tiles, const float4* bias_pre) {
+  constexpr int BR = 256 / BC;  // rows per accumulator group
+  constexpr int TM = BM / (WM * BR);
+  constexpr int TN = BN / (WN * BC);
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
   const int wm = wave / WN, wn = wave % WN;
-  const int lrow = lane & 15;
-  const int g = lane >> 4;
+  const int lcol = lane % BC;
+  const int g = lane / BC;
 
-  // Accumulator element e of lane l in tile (i, j) is row 4*(l/16) + e,
-  // column l%16 of that 16x16 tile.
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j)
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        row_ptr(wm * TM * 16 + i * 16 + g * 4 + e)[wn * TN * 16 + j * 16 + lrow] = acc[i][j][e];
+        row_ptr(wm * TM * BR + i * BR + g * 4 + e)[wn * TN * BC + j * BC + lcol] = acc[i][j][e];
   __syncthreads();
   if (p.splits > 1) {
     // Co is a multiple of 4 for split layers: whole float4 rows.
@@ -695,12 +702,12 @@ __device__ __forceinline__ floatx4 quad_transpose(floatx4 a, int lane) {
 
 // Column group of accumulator block column j of this lane after the quad
 // transpose (finish_regs).
-template <int BN, int WN>
+template <int BN, int WN, int BC = 16>
 __device__ __forceinline__ int regs_col(int n0, int j) {
-  constexpr int TN = BN / (WN * 16);
+  constexpr int TN = BN / (WN * BC);
   const int lane = threadIdx.x & 63;
   const int wn = (threadIdx.x >> 6) % WN;
-  return n0 + wn * TN * 16 + j * 16 + 4 * ((lane & 15) >> 2);
+  return n0 + wn * TN * BC + j * BC + 4 * ((lane % BC) >> 2);
 }
 
 // finish_tile without LDS: the split-K workspace store or the epilogue
@@ -708,11 +715,13 @@ __device__ __forceinline__ int regs_col(int n0, int j) {
 // regs_col(n0, j), loaded ahead.
 // SE: also leave the SE channel sums of the stored output in p.se_part
 // (single-image layers).
-template <typename T, int BM, int BN, int WM, int WN, bool SE = false>
-__device__ __forceinline__ void finish_regs(const ConvParams& p, floatx4 (&acc)[BM / (WM * 16)][BN / (WN * 16)],
-                                            int m0, int n0, int M, const float4 (&bias)[BN / (WN * 16)]) {
-  constexpr int TM = BM / (WM * 16);
-  constexpr int TN = BN / (WN * 16);
+template <typename T, int BM, int BN, int WM, int WN, bool SE = false, int BC = 16>
+__device__ __forceinline__ void finish_regs(const ConvParams& p,
+                                            floatx4 (&acc)[BM * BC / (WM * 256)][BN / (WN * BC)], int m0, int n0, int M,
+                                            const float4 (&bias)[BN / (WN * BC)]) {
+  constexpr int BR = 256 / BC;  // rows per accumulator group
+  constexpr int TM = BM / (WM * BR);
+  constexpr int TN = BN / (WN * BC);
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int wm = wave / WN;
@@ -720,14 +729,14 @@ __device__ __forceinline__ void finish_regs(const ConvParams& p, floatx4 (&acc)[
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j) acc[i][j] = quad_transpose(acc[i][j], lane);
-  const int rsub = 4 * (lane >> 4) + (lane & 3);
+  const int rsub = 4 * (lane / BC) + (lane & 3);
   if (p.splits > 1) {
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
-      const int m = m0 + wm * TM * 16 + i * 16 + rsub;
+      const int m = m0 + wm * TM * BR + i * BR + rsub;
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
-        const int col = regs_col<BN, WN>(n0, j);
+        const int col = regs_col<BN, WN, BC>(n0, j);
         if (m < M && col < p.Co)
           *reinterpret_cast<float4*>(p.split_ws + ((size_t)blockIdx.y * M + m) * p.Co + col) =
               make_float4(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
@@ -747,7 +756,7 @@ __device__ __forceinline__ void finish_regs(const ConvParams& p, floatx4 (&acc)[
   // main loop its occupancy): loads of the block's columns, then the stores.
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
-    const int m = m0 + wm * TM * 16 + i * 16 + rsub;
+    const int m = m0 + wm * TM * BR + i * BR + rsub;
     if (m >= M) continue;
     int img = 0, oy = 0, ox = 0;
     if (need_img) {
@@ -761,12 +770,12 @@ __device__ __forceinline__ void finish_regs(const ConvParams& p, floatx4 (&acc)[
     EpiTerms t[TN];
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
-      const int col = regs_col<BN, WN>(n0, j);
+      const int col = regs_col<BN, WN, BC>(n0, j);
       if (col < p.Co) t[j] = epilogue_load<T>(p, m, col, img, oy, ox);
     }
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
-      const int col = regs_col<BN, WN>(n0, j);
+      const int col = regs_col<BN, WN, BC>(n0, j);
       if (col >= p.Co) continue;
       const float4 v = make_float4(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
       if ((p.Co & 3) != 0) {
@@ -787,15 +796,15 @@ __device__ __forceinline__ void finish_regs(const ConvParams& p, floatx4 (&acc)[
     for (int j = 0; j < TN; ++j) {
       float4 a = se_sum[j];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const int o = k < 2 ? 1 << k : 1 << (k + 2);  // lane bits 0, 1, 4, 5: the rows of a column group
+      for (int o = 1; o < 64; o <<= 1) {
+        if (o >= 4 && o < BC) continue;  // lane bits 0, 1 and those of lane / BC: the rows of a column group
         a.x += __shfl_xor(a.x, o);
         a.y += __shfl_xor(a.y, o);
         a.z += __shfl_xor(a.z, o);
         a.w += __shfl_xor(a.w, o);
       }
-      const int col = regs_col<BN, WN>(n0, j);
-      if ((lane & 0x33) == 0 && col < p.Co)
+      const int col = regs_col<BN, WN, BC>(n0, j);
+      if ((lane & 3) == 0 && lane < BC && col < p.Co)
         *reinterpret_cast<float4*>(p.se_part + ((size_t)(m0 / BM) * WM + wm) * p.Co + col) = a;
     }
   }
@@ -810,12 +819,13 @@ __device__ __forceinline__ void finish_regs(const ConvParams& p, floatx4 (&acc)[
 // float4, free once every wave has passed the barrier), and each (row, tap)
 // item adds its db_ch / 16 blocks in order, applies the sigmoid and writes
 // its 2x2 block of the map (src/cpu/model.rs:1516-1520).
-template <typename T, int BM, int BN, int WM, int WN>
-__device__ __forceinline__ void finish_db_regs(const ConvParams& p, floatx4 (&acc)[BM / (WM * 16)][BN / (WN * 16)],
-                                               int m0, int n0, int M, const float4 (&bias)[BN / (WN * 16)],
-                                               float4* part) {
-  constexpr int TM = BM / (WM * 16);
-  constexpr int TN = BN / (WN * 16);
+template <typename T, int BM, int BN, int WM, int WN, int BC = 16>
+__device__ __forceinline__ void finish_db_regs(const ConvParams& p,
+                                               floatx4 (&acc)[BM * BC / (WM * 256)][BN / (WN * BC)], int m0, int n0,
+                                               int M, const float4 (&bias)[BN / (WN * BC)], float4* part) {
+  constexpr int BR = 256 / BC;  // rows per accumulator group
+  constexpr int TM = BM / (WM * BR);
+  constexpr int TN = BN / (WN * BC);
   constexpr int NB = BN / 16;  // column blocks per tile
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -825,7 +835,7 @@ __device__ __forceinline__ void finish_db_regs(const ConvParams& p, floatx4 (&ac
   float4 wq[TN][4];  // conv_final weights of this lane's four hidden channels per block
 #pragma unroll
   for (int j = 0; j < TN; ++j) {
-    const int o0 = regs_col<BN, WN>(n0, j) % ch;
+    const int o0 = regs_col<BN, WN, BC>(n0, j) % ch;
 #pragma unroll
     for (int e = 0; e < 4; ++e) wq[j][e] = *reinterpret_cast<const float4*>(p.db_wf + (size_t)(o0 + e) * 4);
   }
@@ -833,7 +843,7 @@ __device__ __forceinline__ void finish_db_regs(const ConvParams& p, floatx4 (&ac
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j) acc[i][j] = quad_transpose(acc[i][j], lane);
-  const int rsub = 4 * (lane >> 4) + (lane & 3);
+  const int rsub = 4 * (lane / BC) + (lane & 3);
   float4 f[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
@@ -863,7 +873,7 @@ __device__ __forceinline__ void finish_db_regs(const ConvParams& p, floatx4 (&ac
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int j = 0; j < TN; ++j) part[(wm * TM * 16 + i * 16 + rsub) * NB + wn * TN + j] = f[i][j];
+      for (int j = 0; j < TN; ++j) part[(wm * TM * BR + i * BR + rsub) * NB + (wn * TN + j) * (BC / 16) + (lane % BC) / 16] = f[i][j];
   }
   __syncthreads();
   const int taps = BN / ch, per = ch / 16;
@@ -1360,6 +1370,405 @@ __global__ __launch_bounds__(256) void conv_gemm_direct_multi_kernel(ConvMulti m
 }
 
 // ---------------------------------------------------------------------------
+// fp32 layers on the bf16 matrix cores (p.wt3 set): every fp32 operand is the
+// sum of three bf16 values, x = h + m + l with h = bf16(x), m = bf16(x - h),
+// l = bf16(x - h - m) (24 significant bits, both differences exact), and a
+// product takes the six partial products of weight down to 2^-16,
+// hh + hm + mh + hl + mm + lh, each exact and summed in the MFMA's fp32
+// accumulator: the three-way split of Henry, Tang and Heinecke (2019).  What
+// is left out is below 2^-25 of a product.  Against float64 the sums are
+// closer than the fp32 MFMA's: 2-norm error 1.7e-7, 2.1e-7, 3.0e-7 and 4.1e-7
+// at K = 128, 512, 1024 and 1792 where a chain of fp32 fused multiply-adds
+// leaves 2.1e-7, 3.8e-7, 5.8e-7 and 7.6e-7 (fewer roundings of the running
+// sum: one per 16 products instead of one per product).  Values that round to
+// infinity in bf16 (above 3.38e38) and infinities give NaN.
+//
+// What bounds it: six 32x32x16 MFMAs do the work of eight times as many fp32
+// ones' cycles (2.5 / 6 = 0.42 PFLOP/s against 0.157), and on dense random
+// operands the chip holds about half of that: 165-190 TFLOP/s on the
+// recognizer's K = 512-1024 layers (bf16 MFMA rate 1.0-1.14 PFLOP/s; the
+// library's bf16 product of 8192^3 reaches 1.23), where the fp32 kernel
+// above reaches 120-128.
+//
+// Layout: the weights are split and put in MFMA operand order at load
+// (split3_weights): 1 KB per 32 columns, 16 k values and part, so a wave's
+// operand is one linear 16-byte LDS read per lane and its load from memory
+// one whole KB.  A stays fp32 in memory and in LDS (128-byte rows, one line
+// per row and slice, key direct_key<128>): splitting where the fragment is
+// read costs 11 vector instructions per two values, which run beside the
+// other waves' MFMAs, and no activation is stored wider than before.  In a
+// 16-deep step lane half h holds k = 4h .. 4h + 3 and 8 + 4h .. 8 + 4h + 3
+// (two adjacent 16-byte vectors of the two halves, the read pattern that is
+// conflict-free with this key); the weights are packed in the same order.
+// Two stages of 32-deep slices, the next one loading while one is
+// multiplied; at 64x64 that is 40 KB and four workgroups per CU, which
+// overlap each other's loads, splits and MFMAs (a third stage costs two of
+// the four: 0.75-0.85x).
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kSplitBlock = 32;                                // columns of a weight block
+constexpr unsigned kSplitSlice = 6 * 1024;                     // bytes of a block's 32-deep slice
+constexpr unsigned kSplitStep = 3 * 1024;                      // bytes of a block's 16-deep step
+
+// Eight fp32 values as three bf16 MFMA operands.
+struct Split3 {
+  u32x4 h, m, l;
+};
+__device__ __forceinline__ Split3 split3(floatx4 a, floatx4 b) {
+  const float x[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+  Split3 s;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float x0 = x[2 * i], x1 = x[2 * i + 1];
+    const uint32_t h = pack_bf16x2(x0, x1);
+    const float r0 = x0 - bf16_bits_to_f32(h & 0xFFFFu), r1 = x1 - __builtin_bit_cast(float, h & 0xFFFF0000u);
+    const uint32_t m = pack_bf16x2(r0, r1);
+    const float q0 = r0 - bf16_bits_to_f32(m & 0xFFFFu), q1 = r1 - __builtin_bit_cast(float, m & 0xFFFF0000u);
+    s.h[i] = h;
+    s.m[i] = m;
+    s.l[i] = pack_bf16x2(q0, q1);
+  }
+  return s;
+}
+
+__device__ __forceinline__ floatx16 mfma_32x32(u32x4 a, floatx4 b, floatx16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0,
+                                                 0);
+}
+
+template <int OFF>
+__device__ __forceinline__ floatx4 lds_read16_at(unsigned addr) {
+  floatx4 v;
+  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF));
+  return v;
+}
+
+// Waits until at most N LDS reads of this wave are in flight.
+template <int N>
+__device__ __forceinline__ void lds_wait_to(floatx4& v) {
+  asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(v) : "n"(N));
+}
+
+// PIPE: the second step's operands are read before the first step's MFMAs and
+// split beside them (the tiles that fit two workgroups per CU, where the other
+// workgroup's wave alone does not fill the matrix core: 1.10-1.25x there;
+// even on 64x64).
+template <int BM, int BN, int WM, int WN, bool PW, bool GATE, int EPI, bool PIPE>
+__device__ __forceinline__ void conv_split_tile(const ConvParams& p, int t) {
+  constexpr int BK = 32;
+  constexpr int TM = BM / (WM * 32), TN = BN / (WN * 32);
+  constexpr int AP = BM / 32;                    // A load passes (32 rows each)
+  constexpr int BKB = BN / kSplitBlock * 6;      // 1 KB weight pieces per slice
+  constexpr int BP = (BKB + 3) / 4;              // per wave
+  constexpr int STAGE = BM * 128 + BKB * 1024;
+  constexpr int LDE = BN + 4;
+  static_assert(WM * WN == 4 && TM >= 1 && TN >= 1, "four waves of whole 32x32 blocks");
+  constexpr int STEP_READS = 2 * TM + 3 * TN;
+  static_assert(STEP_READS <= 15, "LDS reads of a step fit the wait count");
+  constexpr int LDS = EPI == EPI_LDS && BM * LDE * 4 > 2 * STAGE ? BM * LDE * 4 : 2 * STAGE;
+  __shared__ __attribute__((aligned(1024))) char lds[LDS];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / WN, wn = wave % WN;
+  const int lrow = lane & 31, half = lane >> 5;
+  const int HoWo = p.Ho * p.Wo;
+  const int M = p.N * HoWo;
+  const int K = p.kh * p.kw * p.C;
+  const int n_tiles = (p.Co + BN - 1) / BN;
+  const int m_tiles = (M + BM - 1) / BM;
+  if (t >= m_tiles * n_tiles) return;
+  const int m0 = (t / n_tiles) * BM;
+  const int n0 = (t % n_tiles) * BN;
+
+  const int nk_all = (K + BK - 1) / BK;
+  const int n_blocks = (p.Co + kSplitBlock - 1) / kSplitBlock;
+  const int32x4_t a_rsrc = buffer_resource(p.in, (unsigned)((size_t)p.N * p.H * p.W * p.in_ps * 4));
+  const int32x4_t b_rsrc = buffer_resource(p.wt3, (unsigned)((size_t)n_blocks * nk_all * kSplitSlice));
+
+  // SE gate of the A rows' images: each lane loads the values of its
+  // fragment's channels with the slice, into registers (in LDS they cost the
+  // fourth workgroup of a CU: 0.87x).
+  int32x4_t g_rsrc{};
+  unsigned g_row[GATE ? TM : 1];
+  if constexpr (GATE) {
+    g_rsrc = buffer_resource(p.in_gate, (unsigned)((size_t)p.N * p.C * 4));
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+      g_row[i] = (unsigned)((size_t)(min(m0 + (wm * TM + i) * 32 + lrow, M - 1) / HoWo) * p.C * 4);
+  }
+
+  // A: this lane fills row pass * 32 + prow, position lane % 8, with k vector
+  // kvec of its source row (kOutOfRange past M); 1x1 layers advance k in the
+  // scalar offset, the others find each slice's tap.
+  const int prow = tid >> 3;
+  const int kvec = (lane & 7) ^ direct_key<128>(prow);
+  unsigned a_off[AP];
+  int a_iy0[AP], a_ix0[AP];
+#pragma unroll
+  for (int i = 0; i < AP; ++i) {
+    const int m = m0 + i * 32 + prow;
+    const bool ok = m < M;
+    const int mm = ok ? m : 0;
+    if constexpr (PW) {
+      a_off[i] = ok ? (unsigned)(((size_t)mm * p.in_ps + kvec * 4) * 4) : kOutOfRange;
+      a_iy0[i] = a_ix0[i] = 0;
+    } else {
+      const int img = mm / HoWo;
+      const int r = mm - img * HoWo;
+      const int oy = r / p.Wo;
+      const int ox = r - oy * p.Wo;
+      a_off[i] = ok ? (unsigned)((size_t)img * p.H * p.W * p.in_ps * 4) : kOutOfRange;
+      a_iy0[i] = oy * p.sh - p.pt;
+      a_ix0[i] = ox * p.sw - p.pl;
+    }
+  }
+  // B: this wave fills pieces wave * BP .. + BP - 1 of the slice (block
+  // piece / 6), each lane its 16 bytes.
+  unsigned b_off[BP];
+#pragma unroll
+  for (int i = 0; i < BP; ++i) {
+    const int piece = wave * BP + i;
+    const int nb = n0 / kSplitBlock + piece / 6;
+    b_off[i] = nb < n_blocks ? (unsigned)nb * (unsigned)nk_all * kSplitSlice + (piece % 6) * 1024 + lane * 16 : kOutOfRange;
+  }
+
+  const int s_begin = (int)((long)blockIdx.y * nk_all / gridDim.y);
+  const int s_end = (int)((long)(blockIdx.y + 1) * nk_all / gridDim.y);
+
+  int kc = s_begin * BK + kvec * 4, kx = 0, ky = 0;
+  if constexpr (!PW) {
+    const int tap = kc / p.C;
+    kc -= tap * p.C;
+    ky = tap / p.kw;
+    kx = tap - ky * p.kw;
+  }
+
+  auto issue = [&](int buf, int s) {
+    char* stage = lds + buf * STAGE;
+    const bool kin = s * BK + kvec * 4 < K;
+#pragma unroll
+    for (int i = 0; i < AP; ++i) {
+      char* dst = stage + (i * 32 + wave * 8) * 128;
+      if constexpr (PW) {
+        lds_load16(a_rsrc, kin ? a_off[i] : kOutOfRange, (unsigned)s * 128u, dst);
+      } else {
+        const int iy = a_iy0[i] + ky;
+        const int ix = a_ix0[i] + kx;
+        const bool ok = kin && a_off[i] != kOutOfRange && (unsigned)iy < (unsigned)p.H && (unsigned)ix < (unsigned)p.W;
+        lds_load16(a_rsrc, ok ? a_off[i] + (unsigned)(((iy * p.W + ix) * p.in_ps + kc) * 4) : kOutOfRange, 0u, dst);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < BP; ++i)
+      if (BKB % 4 == 0 || wave * BP + i < BKB)
+        lds_load16(b_rsrc, b_off[i], (unsigned)s * kSplitSlice, stage + BM * 128 + (wave * BP + i) * 1024);
+    if constexpr (!PW) {
+      kc += BK;
+      while (kc >= p.C) {
+        kc -= p.C;
+        if (++kx == p.kw) {
+          kx = 0;
+          ++ky;
+        }
+      }
+    }
+  };
+
+  floatx16 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+
+  struct Step {
+    floatx4 a0[TM], a1[TM], b[TN][3];
+  };
+  // The gate values of a slice: [step][fragment half].
+  struct Gates {
+    floatx4 v[GATE ? 2 : 1][2][TM];
+  };
+  auto load_gates = [&](int k0, Gates& gt) {
+    if constexpr (GATE) {
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          const int k = k0 + 16 * kk + 8 * q + 4 * half;
+#pragma unroll
+          for (int i = 0; i < TM; ++i)
+            gt.v[kk][q][i] =
+                llvm_raw_buffer_load_v4f32(g_rsrc, k < K ? (int)(g_row[i] + k * 4) : (int)kOutOfRange, 0, 0);
+        }
+    }
+  };
+  const int key = direct_key<128>(lrow);
+  // LDS reads of 16-deep step kk of a stage: 2 TM of A, then 3 TN of B.
+  auto read_step = [&](unsigned stage, int kk, Step& st) {
+    const unsigned a = stage + (wm * TM * 32 + lrow) * 128;
+    const unsigned b = stage + BM * 128 + wn * TN * kSplitSlice + kk * kSplitStep + lane * 16;
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      st.a0[i] = lds_read16(a + i * 32 * 128 + (((4 * kk + half) ^ key) << 4));
+      st.a1[i] = lds_read16(a + i * 32 * 128 + (((4 * kk + 2 + half) ^ key) << 4));
+    }
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      st.b[j][0] = lds_read16_at<0>(b + j * kSplitSlice);
+      st.b[j][1] = lds_read16_at<1024>(b + j * kSplitSlice);
+      st.b[j][2] = lds_read16_at<2048>(b + j * kSplitSlice);
+    }
+  };
+  // Multiplies the A fragments of step kk by their gate values.
+  auto gate_step = [&](const Gates& gt, int kk, Step& st) {
+    if constexpr (GATE) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          st.a0[i][e] = __fmul_rn(st.a0[i][e], gt.v[kk][0][i][e]);
+          st.a1[i][e] = __fmul_rn(st.a1[i][e], gt.v[kk][1][i][e]);
+        }
+    }
+  };
+  auto split_step = [&](const Step& st, Split3 (&sp)[TM]) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i) sp[i] = split3(st.a0[i], st.a1[i]);
+  };
+  // The six partial products, smallest first.
+  auto mfma_step = [&](const Split3 (&sp)[TM], const Step& st) {
+#pragma unroll
+    for (int q = 0; q < 6; ++q)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+          const u32x4 a = q == 0 ? sp[i].l : q == 2 || q == 3 ? sp[i].m : sp[i].h;
+          const floatx4 b = q == 1 ? st.b[j][2] : q == 2 || q == 4 ? st.b[j][1] : st.b[j][0];
+          acc[i][j] = mfma_32x32(a, b, acc[i][j]);
+        }
+  };
+  auto wait_a = [&](Step& st, auto left) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      lds_wait_to<decltype(left)::value>(st.a0[i]);
+      lds_wait_to<decltype(left)::value>(st.a1[i]);
+    }
+  };
+  auto wait_b = [&](Step& st, auto left) {
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int q = 0; q < 3; ++q) lds_wait_to<decltype(left)::value>(st.b[j][q]);
+  };
+  using I0 = std::integral_constant<int, 0>;
+  using IB = std::integral_constant<int, 3 * TN>;
+  using IS = std::integral_constant<int, STEP_READS>;
+  auto compute = [&](int buf, const Gates& gt) {
+    const unsigned stage = lds_addr(lds) + buf * STAGE;
+    if constexpr (PIPE) {
+      Step s0, s1;
+      Split3 p0[TM], p1[TM];
+      read_step(stage, 0, s0);
+      read_step(stage, 1, s1);
+      wait_a(s0, IS{});
+      wait_b(s0, IS{});
+      gate_step(gt, 0, s0);
+      split_step(s0, p0);
+      wait_a(s1, I0{});
+      wait_b(s1, I0{});
+      gate_step(gt, 1, s1);
+      __builtin_amdgcn_s_setprio(1);
+      split_step(s1, p1);
+      mfma_step(p0, s0);
+      mfma_step(p1, s1);
+      __builtin_amdgcn_s_setprio(0);
+    } else {
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk) {
+        Step st;
+        Split3 sp[TM];
+        read_step(stage, kk, st);
+        wait_a(st, IB{});
+        gate_step(gt, kk, st);
+        split_step(st, sp);
+        wait_b(st, I0{});
+        mfma_step(sp, st);
+      }
+    }
+  };
+
+  constexpr bool REGS = EPI != EPI_LDS;
+  constexpr int NB = REGS ? TN : 1;
+  float4 bias_pre[NB];
+#pragma unroll
+  for (int j = 0; j < NB; ++j) {
+    const int bcol = REGS ? regs_col<BN, WN, 32>(n0, j) : staged_col<BN>(n0);
+    bias_pre[j] = p.splits > 1 ? float4{0.f, 0.f, 0.f, 0.f} : bias4(p, bcol);
+    if (REGS && p.splits <= 1 && p.bias && bcol + 1 < p.Co && bcol + 3 >= p.Co)
+      bias_pre[j] = make_float4(p.bias[bcol], p.bias[bcol + 1], 0.f, 0.f);
+  }
+
+  // Slice s is in LDS once every wave has waited for its loads and passed
+  // the barrier, which also says that slice s - 1 is no longer read: its
+  // stage takes slice s + 1.
+  Gates g_cur{}, g_next{};
+  if (s_begin < s_end) {
+    issue(0, s_begin);
+    load_gates(s_begin * BK, g_next);
+  }
+  for (int s = s_begin; s < s_end; ++s) {
+    const int buf = (s - s_begin) & 1;
+    wait_vmcnt<0>();
+    stage_barrier();
+    if constexpr (GATE) g_cur = g_next;
+    if (s + 1 < s_end) {
+      issue(buf ^ 1, s + 1);
+      load_gates((s + 1) * BK, g_next);
+    }
+    compute(buf, g_cur);
+  }
+
+  floatx4 out[4 * TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+        out[4 * i + q][j] =
+            floatx4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+  if constexpr (EPI == EPI_DB) {
+    static_assert(BM * (BN / 16) * 16 <= LDS, "DB partials fit the stages");
+    finish_db_regs<float, BM, BN, WM, WN, 32>(p, out, m0, n0, M, bias_pre, reinterpret_cast<float4*>(lds));
+  } else if constexpr (REGS) {
+    finish_regs<float, BM, BN, WM, WN, EPI == EPI_REGS_SE, 32>(p, out, m0, n0, M, bias_pre);
+  } else {
+    __syncthreads();
+    float* base = reinterpret_cast<float*>(lds);
+    finish_tile<float, BM, BN, WM, WN, 32>(
+        p, out, [=](int row) { return base + row * LDE; }, m0, n0, M, n_tiles, &bias_pre[0]);
+  }
+}
+
+template <int BM, int BN, int WM, int WN, bool PW, bool GATE, int EPI, bool PIPE>
+__global__ __launch_bounds__(256) void conv_split_kernel(ConvParams p) {
+  conv_split_tile<BM, BN, WM, WN, PW, GATE, EPI, PIPE>(p, xcd_tile());
+}
+
+template <int BM, int BN, int WM, int WN, bool PW, int EPI>
+__global__ __launch_bounds__(256) void conv_split_multi_kernel(ConvMulti m) {
+  int t = xcd_tile();
+  int i = 0;
+  while (i + 1 < m.count && t >= m.first[i + 1]) ++i;
+  conv_split_tile<BM, BN, WM, WN, PW, false, EPI, false>(m.p[i], t - m.first[i]);
+}
+
+// ---------------------------------------------------------------------------
 // Wide-tile bf16 1x1 layers (no SE input gate): 256x256 tiles, eight waves
 // (2 x 4) of 128x64 each as 4 x 2 blocks of v_mfma_f32_32x32x16_bf16, so a
 // tile multiplies 8.4 MFLOP per 64 KB K slice it stages: twice the operand
@@ -1393,8 +1802,6 @@ constexpr int kWideBM = 256, kWideBN = 256;
 constexpr int kAuxNontemporal = 2;  // cache-policy bit nt of the buffer load intrinsics
 
 __device__ __forceinline__ int wide_key(int r) { return (r >> 1) & 7; }
-
-typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 // Waits until at most N LDS reads of this wave are in flight; the six
 // operands are the values whose reads must have completed (issued first).
@@ -1889,8 +2296,64 @@ static void launch_tile_kernel(const ConvParams& p, dim3 grid, hipStream_t s) {
   }
 }
 
-template <typename T, int BM, int BN, int WM, int WN>
-static void launch_tile(const ConvParams& p, int M, hipStream_t s) {
+// Tile shapes of the split kernel (conv_split_tile).
+constexpr int kSplitBM[] = {64, 128, 128};
+constexpr int kSplitBN[] = {64, 128, 32};
+constexpr int kSplitWM[] = {2, 2, 4};
+// The 128x128 tile reads ahead (PIPE) and finishes through LDS: its register
+// epilogue does not stay in registers.
+constexpr bool kSplitWide[] = {false, true, false};
+constexpr int kSplitMinTiles = 512;
+constexpr const char* kSplitName[] = {"64x64", "128x128", "128x32"};
+
+// The split kernel's instance for a layer (split_tile).
+template <int I>
+static void launch_split_kernel(const ConvParams& p, dim3 grid, hipStream_t s) {
+  constexpr int BM = kSplitBM[I], BN = kSplitBN[I], WM = kSplitWM[I], WN = 4 / kSplitWM[I];
+  const bool regs = regs_epilogue(p);
+  auto go = [&](auto pw, auto gate, auto epi) {
+    hipLaunchKernelGGL((conv_split_kernel<BM, BN, WM, WN, decltype(pw)::value, decltype(gate)::value,
+                                          decltype(epi)::value, kSplitWide[I]>),
+                       grid, dim3(256), 0, s, p);
+  };
+  using Lds = std::integral_constant<int, EPI_LDS>;
+  using Regs = std::integral_constant<int, EPI_REGS>;
+  using std::false_type;
+  using std::true_type;
+  const int v = conv_variant(p, BM);
+  if constexpr (kSplitWide[I]) {
+    if (v == CV_DIRECT_1X1)
+      go(true_type{}, false_type{}, Lds{});
+    else
+      go(false_type{}, false_type{}, Lds{});
+  } else {
+    if (v == CV_DIRECT_1X1) {
+      if (regs && p.db_ch) {
+        if constexpr (BN == 64) go(true_type{}, false_type{}, std::integral_constant<int, EPI_DB>{});
+      } else if (regs && p.se_part) {
+        go(true_type{}, false_type{}, std::integral_constant<int, EPI_REGS_SE>{});
+      } else if (regs) {
+        go(true_type{}, false_type{}, Regs{});
+      } else {
+        go(true_type{}, false_type{}, Lds{});
+      }
+    } else if (v == CV_DIRECT) {
+      if (regs && !p.db_ch)
+        go(false_type{}, false_type{}, Regs{});
+      else
+        go(false_type{}, false_type{}, Lds{});
+    } else {
+      if (regs && !p.db_ch)
+        go(true_type{}, true_type{}, Regs{});
+      else
+        go(true_type{}, true_type{}, Lds{});
+    }
+  }
+}
+
+template <typename T, typename Launch>
+static void launch_tile(const ConvParams& p, int BM, int BN, hipStream_t s, Launch&& launch) {
+  const int M = p.N * p.Ho * p.Wo;
   // Grid rows of workgroups rounded up to a multiple of the 8 XCDs; surplus
   // workgroups exit before touching memory (see the tile order above).  With
   // split K, grid row y takes split y.  Upsample-on-write layers of short K
@@ -1905,10 +2368,10 @@ static void launch_tile(const ConvParams& p, int M, hipStream_t s) {
   if (p.rep > 1 && splits == 1 && K <= 64 && !p.ctc_part && !p.db_ch) {
     ConvParams q = p;
     q.rep_split = 1;
-    launch_tile_kernel<T, BM, BN, WM, WN>(q, dim3((unsigned)((tiles + 7) / 8 * 8), 1, (unsigned)p.rep), s);
+    launch(q, dim3((unsigned)((tiles + 7) / 8 * 8), 1, (unsigned)p.rep));
     return;
   }
-  launch_tile_kernel<T, BM, BN, WM, WN>(p, dim3((unsigned)((tiles + 7) / 8 * 8), (unsigned)splits), s);
+  launch(p, dim3((unsigned)((tiles + 7) / 8 * 8), (unsigned)splits));
   if (splits > 1) {
     const long fin = (long)((M + kFinishBM - 1) / kFinishBM) * ((p.Co + kFinishBN - 1) / kFinishBN);
     hipLaunchKernelGGL(conv_splitk_finish_kernel<T>, dim3((unsigned)fin), dim3(256), 0, s, p);
@@ -1991,9 +2454,49 @@ static int pick_tile(int M, int cols, int dt) {
   return 3;
 }
 
+// The split kernel's tile for a layer, or -1 where the other kernels run it.
+// Measured against the fp32 kernels in the plans: from 512 tiles (two per CU)
+// 1.0-1.3x; below that the 64x32 fp32 tiles' shorter slices and larger number
+// of workgroups win (299-480 tiles without a split of K 0.7-0.95x, the
+// 40-pixel layers of one line 0.8-0.9x), except where K is deep enough to
+// split (K >= 1024 from 256 tiles: the one-page medium detector's head and
+// stem 3x3 convs 1.29x and 1.24x).  128x128 tiles take K >= 768 layers that
+// leave at least 900 of them (three and a half rounds of two per CU): 1.06-1.10x
+// against 64x64 at K = 768-1024, 0.96-0.99x at K = 512; not the gated
+// layers, whose gate values would cost the second workgroup of a CU, nor
+// those of one image, which may leave SE channel sums from registers.
+static int split_tile(const ConvParams& p) {
+  if (!p.wt3 || p.dt != DT_F32) return -1;
+  const int M = p.N * p.Ho * p.Wo, K = p.kh * p.kw * p.C;
+  const auto tiles = [&](int t) {
+    return (long)((M + kSplitBM[t] - 1) / kSplitBM[t]) * ((p.Co + kSplitBN[t] - 1) / kSplitBN[t]);
+  };
+  int t = p.Co <= 32 ? 2 : 0;
+  if (tiles(t) < kSplitMinTiles && !(K >= 1024 && tiles(t) >= kSplitMinTiles / 2)) return -1;
+  if (K >= 768 && p.Co >= 128 && p.N > 1 && !p.in_gate && !p.db_ch && tiles(1) >= 900) t = 1;
+  const int v = conv_variant(p, kSplitBM[t]);
+  return v == CV_DIRECT_1X1 || v == CV_DIRECT || v == CV_DIRECT_GATE ? t : -1;
+}
+
+// Rows and columns of the tiles launch_conv gives a layer.
+static int tile_rows(const ConvParams& p) {
+  const int t = split_tile(p);
+  return t >= 0 ? kSplitBM[t] : kTileBM[pick_tile(p.N * p.Ho * p.Wo, p.Co, p.dt)];
+}
+static int tile_cols(const ConvParams& p) {
+  const int t = split_tile(p);
+  return t >= 0 ? kSplitBN[t] : kTileBN[pick_tile(p.N * p.Ho * p.Wo, p.Co, p.dt)];
+}
+static long tile_count(const ConvParams& p) {
+  const int bm = tile_rows(p), bn = tile_cols(p);
+  return (long)((p.N * p.Ho * p.Wo + bm - 1) / bm) * ((p.Co + bn - 1) / bn);
+}
+
 std::string conv_kernel_name(const ConvParams& p) {
   if (wide_layer(p)) return "conv_gemm_bf16<256x256,1x1>";
   static const char* variants[] = {",1x1", "", ",1x1,gate", ",1x1,reg", ",reg", ",1x1,reg4", ",reg4"};
+  if (const int st = split_tile(p); st >= 0)
+    return std::string("conv_split<") + kSplitName[st] + variants[conv_variant(p, kSplitBM[st])] + ">";
   const int t = pick_tile(p.N * p.Ho * p.Wo, p.Co, p.dt);
   const int v = conv_variant(p, kTileBM[t]);
   const bool r128 = t == 3 && ((v == CV_DIRECT_1X1 && rows128_layer(p)) || (v == CV_DIRECT && rows128_kxk(p)));
@@ -2006,14 +2509,13 @@ int conv_se_blocks(const ConvParams& p) {
       !regs_epilogue(p))
     return 0;
   const int M = p.Ho * p.Wo;
-  const int t = pick_tile(M, p.Co, p.dt);
-  if (conv_variant(p, kTileBM[t]) != CV_DIRECT_1X1) return 0;
-  return (M + kTileBM[t] - 1) / kTileBM[t] * kTileWM[t];
+  const int bm = tile_rows(p);
+  if (conv_variant(p, bm) != CV_DIRECT_1X1) return 0;
+  const int st = split_tile(p);
+  return (M + bm - 1) / bm * (st >= 0 ? kSplitWM[st] : kTileWM[pick_tile(M, p.Co, p.dt)]);
 }
 
-int conv_tile_cols(int M, int cols, int dt) {
-  return kTileBN[pick_tile(M, cols, dt)];
-}
+int conv_tile_cols(const ConvParams& p) { return tile_cols(p); }
 
 // Split K when the tiles fill fewer than 192 of the 256 CUs: enough splits
 // for about two workgroups per CU.  Also when they give only one to two
@@ -2030,13 +2532,17 @@ int conv_tile_cols(int M, int cols, int dt) {
 // 7 ways 0.96x).  Each split keeps at
 // least 8 K slices (the load pipeline is 3-4 slices deep), at most 16
 // splits.
-int conv_split_k(int M, int Co, int K, int dt) {
-  const int t = pick_tile(M, Co, dt);
-  const long tiles = (long)((M + kTileBM[t] - 1) / kTileBM[t]) * ((Co + kTileBN[t] - 1) / kTileBN[t]);
-  const int bk = dt == DT_BF16 ? GemmTraits<bf16>::BK : GemmTraits<float>::BK;
-  const int nk = (K + bk - 1) / bk;
+int conv_split_k(const ConvParams& p) {
+  const int M = p.N * p.Ho * p.Wo, Co = p.Co, K = p.kh * p.kw * p.C, dt = p.dt;
+  const long tiles = tile_count(p);
   if (Co % 4 != 0 || wide_shape(M, Co, K, dt)) return 1;
   long s;
+  if (split_tile(p) >= 0) {
+    // Only the deep layers below kSplitMinTiles: three workgroups per CU.
+    return tiles < kSplitMinTiles ? (int)std::min<long>((768 + tiles - 1) / tiles, kMaxSplits) : 1;
+  }
+  const int bk = dt == DT_BF16 ? GemmTraits<bf16>::BK : GemmTraits<float>::BK;
+  const int nk = (K + bk - 1) / bk;
   if (tiles < 192)
     s = (512 + tiles - 1) / tiles;
   else if (tiles <= (dt == DT_F32 ? 640 : 560) && nk >= 48)
@@ -2049,8 +2555,16 @@ int conv_split_k(int M, int Co, int K, int dt) {
 }
 
 template <typename T, int I>
-static void launch_tile_shape(const ConvParams& p, int M, hipStream_t s) {
-  launch_tile<T, kTileBM[I], kTileBN[I], kTileWM[I], 4 / kTileWM[I]>(p, M, s);
+static void launch_tile_shape(const ConvParams& p, hipStream_t s) {
+  launch_tile<T>(p, kTileBM[I], kTileBN[I], s, [&](const ConvParams& q, dim3 grid) {
+    launch_tile_kernel<T, kTileBM[I], kTileBN[I], kTileWM[I], 4 / kTileWM[I]>(q, grid, s);
+  });
+}
+
+template <int I>
+static void launch_split_shape(const ConvParams& p, hipStream_t s) {
+  launch_tile<float>(p, kSplitBM[I], kSplitBN[I], s,
+                     [&](const ConvParams& q, dim3 grid) { launch_split_kernel<I>(q, grid, s); });
 }
 
 int device_cus() {
@@ -2067,9 +2581,9 @@ int device_cus() {
 
 template <typename T>
 static void launch_typed(const ConvParams& p, hipStream_t s) {
-  int M = p.N * p.Ho * p.Wo;
   if constexpr (sizeof(T) == 2) {
     if (wide_layer(p)) {
+      const int M = p.N * p.Ho * p.Wo;
       // One persistent workgroup per CU (a multiple of 8, one share per XCD).
       const long tiles = (long)((M + kWideBM - 1) / kWideBM) * ((p.Co + kWideBN - 1) / kWideBN);
       const dim3 grid((unsigned)std::min<long>((tiles + 7) / 8 * 8, std::max(8, device_cus() / 8 * 8)));
@@ -2099,14 +2613,62 @@ static void launch_typed(const ConvParams& p, hipStream_t s) {
       return;
     }
   }
-  switch (pick_tile(M, p.Co, p.dt)) {
-    case 0: launch_tile_shape<T, 0>(p, M, s); break;
-    case 1: launch_tile_shape<T, 1>(p, M, s); break;
-    case 2: launch_tile_shape<T, 2>(p, M, s); break;
-    case 3: launch_tile_shape<T, 3>(p, M, s); break;
-    case 4: launch_tile_shape<T, 4>(p, M, s); break;
-    default: launch_tile_shape<T, 5>(p, M, s); break;
+  if constexpr (sizeof(T) == 4) {
+    switch (split_tile(p)) {
+      case 0: launch_split_shape<0>(p, s); return;
+      case 1: launch_split_shape<1>(p, s); return;
+      case 2: launch_split_shape<2>(p, s); return;
+      default: break;
+    }
   }
+  switch (pick_tile(p.N * p.Ho * p.Wo, p.Co, p.dt)) {
+    case 0: launch_tile_shape<T, 0>(p, s); break;
+    case 1: launch_tile_shape<T, 1>(p, s); break;
+    case 2: launch_tile_shape<T, 2>(p, s); break;
+    case 3: launch_tile_shape<T, 3>(p, s); break;
+    case 4: launch_tile_shape<T, 4>(p, s); break;
+    default: launch_tile_shape<T, 5>(p, s); break;
+  }
+}
+
+bool conv_takes_split3(int Co, int K) {
+  return Co >= 24 && K >= 64 && split3_size(Co, K) * 2 < kOutOfRange;
+}
+
+size_t split3_size(int Co, int K) {
+  return (size_t)((Co + kSplitBlock - 1) / kSplitBlock) * ((K + 31) / 32) * (kSplitSlice / 2);
+}
+
+static uint16_t bf16_rne(float f) {
+  uint32_t u;
+  memcpy(&u, &f, 4);
+  return (u & 0x7FFFFFFFu) > 0x7F800000u ? (uint16_t)((u >> 16) | 0x40u)
+                                          : (uint16_t)((u + 0x7FFFu + ((u >> 16) & 1u)) >> 16);
+}
+static float bf16_widen(uint16_t h) {
+  const uint32_t u = (uint32_t)h << 16;
+  float f;
+  memcpy(&f, &u, 4);
+  return f;
+}
+
+// Value k of column n: block n / 32, step k / 16, part (h, m, l), lane
+// 32 half + n % 32 with half = (k / 4) % 2, element 4 ((k % 16) / 8) + k % 4.
+void split3_weights(const float* w, int Co, int K, uint16_t* out) {
+  const size_t steps = (size_t)((K + 31) / 32) * 2;
+  memset(out, 0, split3_size(Co, K) * 2);
+  for (int n = 0; n < Co; ++n)
+    for (int k = 0; k < K; ++k) {
+      const float x = w[(size_t)n * K + k];
+      const uint16_t h = bf16_rne(x);
+      const float r = x - bf16_widen(h);
+      const uint16_t m = bf16_rne(r);
+      uint16_t* o = out + (((size_t)(n / 32) * steps + k / 16) * 3) * 512 +
+                    (size_t)(((k >> 2) & 1) * 32 + n % 32) * 8 + ((k >> 3) & 1) * 4 + (k & 3);
+      o[0] = h;
+      o[512] = m;
+      o[1024] = bf16_rne(r - bf16_widen(m));
+    }
 }
 
 bool conv_multi_supported(const ConvParams* p, int count) {
@@ -2114,9 +2676,9 @@ bool conv_multi_supported(const ConvParams* p, int count) {
   const std::string name = conv_kernel_name(p[0]);
   for (int i = 0; i < count; ++i) {
     const ConvParams& q = p[i];
-    const int t = pick_tile(q.N * q.Ho * q.Wo, q.Co, q.dt);
-    const int v = conv_variant(q, kTileBM[t]);
+    const int v = conv_variant(q, tile_rows(q));
     if (q.dt != p[0].dt || q.splits > 1 || q.rep != 1 || q.db_ch || q.ctc_part || q.in_gate || wide_layer(q) ||
+        split_tile(q) == 1 ||
         (v != CV_DIRECT_1X1 && v != CV_DIRECT) || conv_kernel_name(q) != name ||
         regs_epilogue(q) != regs_epilogue(p[0]) || (q.se_part != nullptr) != (p[0].se_part != nullptr))
       return false;
@@ -2170,16 +2732,43 @@ static void launch_multi_kernel(const ConvMulti& m, dim3 grid, hipStream_t s) {
   }
 }
 
-template <typename T>
-static void launch_multi_typed(const ConvMulti& m, hipStream_t s) {
-  const int t = pick_tile(m.p[0].N * m.p[0].Ho * m.p[0].Wo, m.p[0].Co, m.p[0].dt);
-  long total = 0;
-  for (int i = 0; i < m.count; ++i) {
-    const ConvParams& q = m.p[i];
-    total += (long)((q.N * q.Ho * q.Wo + kTileBM[t] - 1) / kTileBM[t]) * ((q.Co + kTileBN[t] - 1) / kTileBN[t]);
+// Small layers share a launch, so never the 128x128 tile.
+template <int I>
+static void launch_split_multi(const ConvMulti& m, dim3 grid, hipStream_t s) {
+  constexpr int BM = kSplitBM[I], BN = kSplitBN[I], WM = kSplitWM[I], WN = 4 / kSplitWM[I];
+  const ConvParams& p = m.p[0];
+  auto go = [&](auto pw, auto epi) {
+    hipLaunchKernelGGL((conv_split_multi_kernel<BM, BN, WM, WN, decltype(pw)::value, decltype(epi)::value>), grid,
+                       dim3(256), 0, s, m);
+  };
+  using Lds = std::integral_constant<int, EPI_LDS>;
+  using Regs = std::integral_constant<int, EPI_REGS>;
+  const bool regs = regs_epilogue(p);
+  if (conv_variant(p, BM) == CV_DIRECT_1X1) {
+    if (regs && p.se_part)
+      go(std::true_type{}, std::integral_constant<int, EPI_REGS_SE>{});
+    else if (regs)
+      go(std::true_type{}, Regs{});
+    else
+      go(std::true_type{}, Lds{});
+  } else {
+    if (regs)
+      go(std::false_type{}, Regs{});
+    else
+      go(std::false_type{}, Lds{});
   }
-  const dim3 grid((unsigned)((total + 7) / 8 * 8));
-  switch (t) {
+}
+
+template <typename T>
+static void launch_multi_typed(const ConvMulti& m, dim3 grid, hipStream_t s) {
+  if constexpr (sizeof(T) == 4) {
+    switch (split_tile(m.p[0])) {
+      case 0: launch_split_multi<0>(m, grid, s); return;
+      case 2: launch_split_multi<2>(m, grid, s); return;
+      default: break;
+    }
+  }
+  switch (pick_tile(m.p[0].N * m.p[0].Ho * m.p[0].Wo, m.p[0].Co, m.p[0].dt)) {
     case 0: launch_multi_kernel<T, kTileBM[0], kTileBN[0], kTileWM[0], 4 / kTileWM[0]>(m, grid, s); break;
     case 1: launch_multi_kernel<T, kTileBM[1], kTileBN[1], kTileWM[1], 4 / kTileWM[1]>(m, grid, s); break;
     case 2: launch_multi_kernel<T, kTileBM[2], kTileBN[2], kTileWM[2], 4 / kTileWM[2]>(m, grid, s); break;
@@ -2192,17 +2781,16 @@ static void launch_multi_typed(const ConvMulti& m, hipStream_t s) {
 void launch_conv_multi(const ConvMulti& mm, hipStream_t s) {
   if (!conv_multi_supported(mm.p, mm.count)) throw std::runtime_error("launch_conv_multi: layers cannot share a launch");
   ConvMulti m = mm;
-  const int t = pick_tile(m.p[0].N * m.p[0].Ho * m.p[0].Wo, m.p[0].Co, m.p[0].dt);
   int first = 0;
   for (int i = 0; i < m.count; ++i) {
-    const ConvParams& q = m.p[i];
     m.first[i] = first;
-    first += ((q.N * q.Ho * q.Wo + kTileBM[t] - 1) / kTileBM[t]) * ((q.Co + kTileBN[t] - 1) / kTileBN[t]);
+    first += (int)tile_count(m.p[i]);
   }
+  const dim3 grid((unsigned)((first + 7) / 8 * 8));
   if (m.p[0].dt == DT_BF16)
-    launch_multi_typed<bf16>(m, s);
+    launch_multi_typed<bf16>(m, grid, s);
   else
-    launch_multi_typed<float>(m, s);
+    launch_multi_typed<float>(m, grid, s);
 }
 
 void launch_conv(const ConvParams& p, hipStream_t s) {

@@ -42,6 +42,7 @@ struct ConvParams {
   int Ho, Wo, Co, out_ps;
   const void* wt;  // packed [Co][ldw] in the activation type
   int ldw;         // = K (a multiple of 4)
+  const void* wt3;  // the same weights split for the bf16 matrix cores (split3_weights), fp32 layers; null: not split
   const float* bias;  // [Co] or null
   int kh, kw, sh, sw, pt, pl;
   int act;
@@ -248,14 +249,19 @@ void launch_pointwise_pair(const PairParams& p, hipStream_t s);
 // for null and 16-byte alignment.
 std::string conv_kernel_name(const ConvParams& p);
 // Column width of that instance's tiles.
-int conv_tile_cols(int M, int cols, int dt);
+int conv_tile_cols(const ConvParams& p);
+// fp32 weights [Co][K] (K along a row) as the three-part bf16 operands of the
+// split conv kernel: split3_size() 16-bit values, zero past Co and K.
+bool conv_takes_split3(int Co, int K);  // layers the split kernel can run
+size_t split3_size(int Co, int K);
+void split3_weights(const float* w, int Co, int K, uint16_t* out);
 // Rows of the SE channel-sum array the conv leaves in se_part (single-image
 // fp32 1x1 layers finished from registers), or 0 where it cannot.
 int conv_se_blocks(const ConvParams& p);
-// K splits for a convolution of M rows, Co columns and reduction depth K:
-// more than 1 when its tiles alone would leave most of the 256 CUs idle and
-// K is deep enough to divide (the workspace is splits * M * Co floats).
-int conv_split_k(int M, int Co, int K, int dt);
+// K splits for a convolution (M rows, Co columns): more than 1 when its tiles
+// alone would leave most of the 256 CUs idle and K is deep enough to divide
+// (the workspace is splits * M * Co floats).
+int conv_split_k(const ConvParams& p);
 // Merges the greedy-CTC partials of launch_conv into one (class, probability)
 // pair per row: out[m] = {argmax (ties -> last index), softmax value of it}.
 void launch_ctc_merge(const float* part, int M, int n_tiles, float* out, hipStream_t s);

@@ -41,6 +41,7 @@ float bf16_value(float f) {
 
 struct ConvW {
   size_t w = NOW, b = NOW;  // byte offsets into the weight blob
+  size_t w3 = NOW;          // the weights split for the bf16 matrix cores (fp32 plans)
   int ldw = 0;
   int ci = 0, ci_pad = 0, co = 0, kh = 1, kw = 1, sh = 1, sw = 1, pt = 0, pl = 0, pb = 0, pr = 0;
 };
@@ -146,6 +147,12 @@ class Builder {
           for (int kx = 0; kx < kw; ++kx)
             packed[(size_t)o * K + (size_t)(ky * kw + kx) * c.ci_pad + i] = W[(((size_t)o * ci + i) * kh + ky) * kw + kx];
     c.w = put_act(packed);
+    if (dt_ == DT_F32 && conv_takes_split3(co, (int)K)) {
+      const size_t n = split3_size(co, (int)K);
+      c.w3 = round_up(plan_.weights.size(), 256);
+      plan_.weights.resize(c.w3 + n * 2);
+      split3_weights(packed.data(), co, (int)K, reinterpret_cast<uint16_t*>(plan_.weights.data() + c.w3));
+    }
     if (!b.empty()) c.b = put(b);
     return c;
   }
@@ -259,16 +266,18 @@ class Builder {
   // will pass (kTermRes, kTermResGate, kTermUp, kTermCtc), stood in for by
   // non-null aligned values.
   static constexpr unsigned kTermRes = 1, kTermResGate = 2, kTermUp = 4, kTermCtc = 8;
-  static std::string conv_kernel(const ConvParams& base, const View& x, size_t wo, bool gated, unsigned terms = 0) {
-    return conv_kernel_name(stand_in(base, x, wo, gated, terms));
+  static std::string conv_kernel(const ConvParams& base, const View& x, const ConvW& w, bool gated,
+                                 unsigned terms = 0) {
+    return conv_kernel_name(stand_in(base, x, w, gated, terms));
   }
   // `base` with its pointers stood in for as above.
-  static ConvParams stand_in(const ConvParams& base, const View& x, size_t wo, bool gated, unsigned terms) {
+  static ConvParams stand_in(const ConvParams& base, const View& x, const ConvW& w, bool gated, unsigned terms) {
     ConvParams probe = base;
-    probe.in = reinterpret_cast<const void*>((uintptr_t)(x.off * dtype_size(x.dt)));
-    probe.wt = reinterpret_cast<const void*>((uintptr_t)wo);
-    probe.in_gate = gated ? reinterpret_cast<const float*>((uintptr_t)16) : nullptr;
     const uintptr_t nonnull = 256;
+    probe.in = reinterpret_cast<const void*>((uintptr_t)(x.off * dtype_size(x.dt)));
+    probe.wt = reinterpret_cast<const void*>((uintptr_t)w.w);
+    probe.wt3 = w.w3 == NOW ? nullptr : reinterpret_cast<const void*>(nonnull);
+    probe.in_gate = gated ? reinterpret_cast<const float*>((uintptr_t)16) : nullptr;
     if (terms & kTermRes) probe.res = reinterpret_cast<const void*>(nonnull);
     if (terms & kTermResGate) probe.res_gate = reinterpret_cast<const float*>(nonnull);
     if (terms & kTermUp) probe.up = reinterpret_cast<const void*>(nonnull);
@@ -342,9 +351,9 @@ class Builder {
     base.rep = e.rep;
     base.out_h = oh, base.out_w = ow;
     base.dt = x.dt;
-    size_t wo = w.w, bo = w.b;
+    size_t wo = w.w, bo = w.b, wo3 = w.w3;
     // Split-K workspace [splits][M][Co] fp32, live for this op only.
-    const int splits = conv_split_k(x.n * Ho * Wo, w.co, w.kh * w.kw * x.c, x.dt);
+    const int splits = conv_split_k(stand_in(base, a_src, w, has_ig && !prescale, 0));
     View ws;
     if (splits > 1) ws = alloc(1, splits, x.n * Ho * Wo, w.co, name + ".split_k", DT_F32);
     base.splits = splits;
@@ -353,7 +362,7 @@ class Builder {
     bool has_part = false;
     if (sp) {
       sp->P = 0;
-      const int P = conv_se_blocks(stand_in(base, a_src, wo, has_ig && !prescale, terms));
+      const int P = conv_se_blocks(stand_in(base, a_src, w, has_ig && !prescale, terms));
       if (P > 0) {
         part = alloc(1, P, 1, w.co, name + ".se_partial", DT_F32);
         has_part = true;
@@ -364,7 +373,7 @@ class Builder {
     Op op;
     op.name = name;
     if (dt_ == DT_BF16) op.bf16_weights = {name};
-    op.kernel = conv_kernel(base, a_src, wo, has_ig && !prescale, terms);
+    op.kernel = conv_kernel(base, a_src, w, has_ig && !prescale, terms);
     if (prescale) op.kernel += "+gate_pass";
     if (splits > 1) op.kernel += "+split_k" + std::to_string(splits);
     op.bound = 1;
@@ -391,6 +400,7 @@ class Builder {
       p.in_gate = has_ig && !prescale ? ex.fptr(ig) : nullptr;
       p.out = ex.ptr(out);
       p.wt = ex.wv(wo);
+      p.wt3 = ex.wv(wo3);
       p.bias = ex.w(bo);
       p.res = has_res ? ex.ptr(res) : nullptr;
       p.res_gate = has_rg ? ex.fptr(rg) : nullptr;
@@ -405,7 +415,7 @@ class Builder {
       launch_conv(fill(ex), s);
     };
     if (defer) {
-      ConvParams shape = stand_in(base, a_src, wo, has_ig && !prescale, terms);
+      ConvParams shape = stand_in(base, a_src, w, has_ig && !prescale, terms);
       shape.splits = splits;
       shape.se_part = has_part ? reinterpret_cast<float*>((uintptr_t)256) : nullptr;
       *defer = Deferred{std::move(op), fill, shape};
@@ -1023,11 +1033,6 @@ class Builder {
       raise(PPOCR_ERR_INVALID_MODEL, name + ": greedy classifier takes [N, 1, T, C] rows");
     if (w.b == NOW) raise(PPOCR_ERR_INVALID_MODEL, name + ": classifier needs a bias");
     const int M = x.n * x.w;
-    const int bn = conv_tile_cols(M, w.co, x.dt);
-    const int tiles = (w.co + bn - 1) / bn;
-    if ((size_t)3 * tiles * M > (size_t)INT32_MAX) raise(PPOCR_ERR_INVALID_INPUT, name + ": batch too large");
-    View part = alloc(1, 1, 1, 3 * tiles * M, name + ".partials", DT_F32);
-    View out = alloc(x.n, 1, x.w, 2, "output", DT_F32);
     ConvParams base{};
     base.N = x.n, base.H = 1, base.W = x.w, base.C = x.c, base.in_ps = x.ps;
     base.Ho = 1, base.Wo = x.w, base.Co = w.co, base.out_ps = 0;
@@ -1038,12 +1043,17 @@ class Builder {
     base.rep = 1;
     base.out_h = 1, base.out_w = x.w;
     base.dt = x.dt;
+    const int bn = conv_tile_cols(stand_in(base, x, w, false, kTermCtc));
+    const int tiles = (w.co + bn - 1) / bn;
+    if ((size_t)3 * tiles * M > (size_t)INT32_MAX) raise(PPOCR_ERR_INVALID_INPUT, name + ": batch too large");
+    View part = alloc(1, 1, 1, 3 * tiles * M, name + ".partials", DT_F32);
+    View out = alloc(x.n, 1, x.w, 2, "output", DT_F32);
     const View in = x;
-    const size_t wo = w.w, bo = w.b;
+    const size_t wo = w.w, wo3 = w.w3, bo = w.b;
     const double es = (double)dtype_size(x.dt), part_bytes = 12.0 * tiles * M;
     Op op;
     op.name = name;
-    op.kernel = conv_kernel(base, x, wo, false, kTermCtc);
+    op.kernel = conv_kernel(base, x, w, false, kTermCtc);
     op.bound = 1;
     op.flops = 2.0 * M * w.co * w.ci;
     op.bytes = es * ((double)M * w.ci + (double)w.ci * w.co) + 4.0 * w.co + part_bytes;
@@ -1054,6 +1064,7 @@ class Builder {
       p.in = ex.ptr(in);
       p.out = nullptr;
       p.wt = ex.wv(wo);
+      p.wt3 = ex.wv(wo3);
       p.bias = ex.w(bo);
       p.ctc_part = ex.fptr(part);
       launch_conv(p, s);
@@ -1555,8 +1566,23 @@ void detector_head(Builder& B, const View& x, int nc) {
   op.bytes = (double)dtype_size(d.dt) * d.pixels() * h + 4.0 * ((double)out.pixels() + 4.0 * h * h + 4.0 * h);
   op.reads = {d.buf};
   op.writes = {out.buf};
-  const int M = d.n * d.h * d.w;
-  if (conv_tile_cols(M, 4 * h, d.dt) % h == 0) {
+  ConvParams base{};
+  base.N = d.n, base.H = d.h, base.W = d.w, base.C = d.c, base.in_ps = d.ps;
+  base.Ho = d.h, base.Wo = d.w, base.Co = 4 * h, base.out_ps = 1;
+  base.out_f32 = 1;
+  base.ldw = h;
+  base.kh = base.kw = base.sh = base.sw = 1;
+  base.act = ACT_RELU;
+  base.up_s = 2;
+  base.rep = 1;
+  base.out_h = out.h, base.out_w = out.w;
+  base.dt = d.dt;
+  base.db_ch = h;
+  base.db_bf = bf;
+  ConvW shape;
+  shape.w = 0;
+  if (B.dt() == DT_F32 && conv_takes_split3(4 * h, h)) shape.w3 = 0;
+  if (conv_tile_cols(Builder::stand_in(base, d, shape, false, 0)) % h == 0) {
     // conv_up on the matrix cores as a 1x1 conv with 4h columns (column
     // tap * h + o, weight wu[c][o][tap], bias bu[o]); conv_final and the
     // sigmoid run in its epilogue (tiles are whole taps wide).
@@ -1567,27 +1593,15 @@ void detector_head(Builder& B, const View& x, int nc) {
         for (int c = 0; c < h; ++c) w1[((size_t)tap * h + o) * h + c] = wu[((size_t)c * h + o) * 4 + tap];
       }
     const ConvW up = B.pack_conv(w1, b1, h, 4 * h, 1, 1, 1, 1, {0, 0, 0, 0});
-    ConvParams base{};
-    base.N = d.n, base.H = d.h, base.W = d.w, base.C = d.c, base.in_ps = d.ps;
-    base.Ho = d.h, base.Wo = d.w, base.Co = 4 * h, base.out_ps = 1;
-    base.out_f32 = 1;
-    base.ldw = up.ldw;
-    base.kh = base.kw = base.sh = base.sw = 1;
-    base.act = ACT_RELU;
-    base.up_s = 2;
-    base.rep = 1;
-    base.out_h = out.h, base.out_w = out.w;
-    base.dt = d.dt;
-    base.db_ch = h;
-    base.db_bf = bf;
-    const size_t uw = up.w, ub = up.b;
-    op.kernel = Builder::conv_kernel(base, d, uw, false) + "+db_head";
+    const size_t uw = up.w, uw3 = up.w3, ub = up.b;
+    op.kernel = Builder::conv_kernel(base, d, up, false) + "+db_head";
     op.bound = 1;
     op.launch = [=](const Exec& ex, hipStream_t s) {
       ConvParams p = base;
       p.in = ex.ptr(in);
       p.out = ex.fptr(out);
       p.wt = ex.wv(uw);
+      p.wt3 = ex.wv(uw3);
       p.bias = ex.w(ub);
       p.db_wf = ex.w(owf);
       launch_conv(p, s);

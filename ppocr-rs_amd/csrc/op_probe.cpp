@@ -46,9 +46,10 @@ void* upload(const float* src, size_t n, int dt) {
 
 // ppocr_probe_conv, and with se_rows the SE channel sums the conv leaves:
 // *se_rows = conv_se_blocks() and se_part [*se_rows][co] (when non-zero).
+// With split3 the layer also has its weights split for the bf16 matrix cores.
 int run_conv(const float* x, int n, int h, int w, int c, const float* weight, const float* bias, int co, int kh,
              int kw, int sh, int sw, int pt, int pl, int pb, int pr, int act, const float* gate, int splits, int dt,
-             float* out, int* se_rows, float* se_part) {
+             float* out, int* se_rows, float* se_part, bool split3 = false, std::string* kernel = nullptr) {
   const int ho = (h + pt + pb - kh) / sh + 1, wo = (w + pl + pr - kw) / sw + 1;
   const size_t K = (size_t)kh * kw * c, M = (size_t)n * ho * wo;
   std::vector<float> packed((size_t)co * K);
@@ -61,10 +62,17 @@ int run_conv(const float* x, int n, int h, int w, int c, const float* weight, co
   void* d_wt = upload(packed.data(), packed.size(), dt);
   void* d_bias = bias ? upload(bias, co, ppocr::DT_F32) : nullptr;
   void* d_gate = gate ? upload(gate, (size_t)n * c, ppocr::DT_F32) : nullptr;
-  void *d_out = nullptr, *d_ws = nullptr, *d_se = nullptr;
+  void *d_out = nullptr, *d_ws = nullptr, *d_se = nullptr, *d_wt3 = nullptr;
   int rc = 0;
   const size_t es = dt == ppocr::DT_BF16 ? 2 : 4;
-  if (!d_in || !d_wt || (bias && !d_bias) || (gate && !d_gate) || hipMalloc(&d_out, M * co * es) != hipSuccess ||
+  if (split3) {
+    std::vector<uint16_t> parts(ppocr::split3_size(co, (int)K));
+    ppocr::split3_weights(packed.data(), co, (int)K, parts.data());
+    if (hipMalloc(&d_wt3, parts.size() * 2) != hipSuccess ||
+        hipMemcpy(d_wt3, parts.data(), parts.size() * 2, hipMemcpyHostToDevice) != hipSuccess)
+      rc = 1;
+  }
+  if (rc || !d_in || !d_wt || (bias && !d_bias) || (gate && !d_gate) || hipMalloc(&d_out, M * co * es) != hipSuccess ||
       (splits > 1 && hipMalloc(&d_ws, (size_t)splits * M * co * 4) != hipSuccess)) {
     rc = 1;
   } else {
@@ -74,6 +82,7 @@ int run_conv(const float* x, int n, int h, int w, int c, const float* weight, co
     p.out = d_out;
     p.Ho = ho, p.Wo = wo, p.Co = co, p.out_ps = co;
     p.wt = d_wt;
+    p.wt3 = d_wt3;
     p.ldw = (int)K;
     p.bias = static_cast<const float*>(d_bias);
     p.kh = kh, p.kw = kw, p.sh = sh, p.sw = sw, p.pt = pt, p.pl = pl;
@@ -90,6 +99,7 @@ int run_conv(const float* x, int n, int h, int w, int c, const float* weight, co
       if (*se_rows > 0 && hipMalloc(&d_se, (size_t)*se_rows * co * 4) != hipSuccess) rc = 1;
       p.se_part = static_cast<float*>(d_se);
     }
+    if (kernel) *kernel = ppocr::conv_kernel_name(p);
     if (rc == 0) {
       ppocr::launch_conv(p, nullptr);
       if (hipDeviceSynchronize() != hipSuccess) rc = 1;
@@ -106,7 +116,7 @@ int run_conv(const float* x, int n, int h, int w, int c, const float* weight, co
       }
     }
   }
-  for (void* ptr : {d_in, d_wt, d_bias, d_gate, d_out, d_ws, d_se})
+  for (void* ptr : {d_in, d_wt, d_bias, d_gate, d_out, d_ws, d_se, d_wt3})
     if (ptr) (void)hipFree(ptr);
   return rc;
 }
@@ -191,6 +201,24 @@ int ppocr_probe_conv(const float* x, int n, int h, int w, int c, const float* we
                      int splits, int dt, float* out) {
   return run_conv(x, n, h, w, c, weight, bias, co, kh, kw, sh, sw, pt, pl, pb, pr, act, gate, splits, dt, out,
                   nullptr, nullptr);
+}
+
+// ppocr_probe_conv of an fp32 layer whose weights are also split for the bf16
+// matrix cores; *kernel: the instance that ran.
+int ppocr_probe_conv_split3(const float* x, int n, int h, int w, int c, const float* weight, const float* bias, int co,
+                            int kh, int kw, int sh, int sw, int pt, int pl, int pb, int pr, int act, const float* gate,
+                            int splits, float* out, int* se_rows, float* se_part, const char** kernel) {
+  static thread_local std::string name;
+  const int rc = run_conv(x, n, h, w, c, weight, bias, co, kh, kw, sh, sw, pt, pl, pb, pr, act, gate, splits,
+                          ppocr::DT_F32, out, se_rows, se_part, true, &name);
+  *kernel = name.c_str();
+  return rc;
+}
+
+// The packed parts of split3_weights for weight [co][k].
+size_t ppocr_probe_split3_size(int co, int k) { return ppocr::split3_size(co, k); }
+void ppocr_probe_split3_weights(const float* weight, int co, int k, uint16_t* out) {
+  ppocr::split3_weights(weight, co, k, out);
 }
 
 // ppocr_probe_conv without K splits, also asking for the squeeze-excitation
@@ -322,7 +350,7 @@ const char* ppocr_probe_conv_kernel(int n, int h, int w, int c, int co, int kh, 
   p.in_gate = gated ? reinterpret_cast<const float*>((uintptr_t)256) : nullptr;
   p.dt = dt;
   name = ppocr::conv_kernel_name(p);
-  if (planner_splits) *planner_splits = ppocr::conv_split_k(n * ho * wo, co, kh * kw * c, dt);
+  if (planner_splits) *planner_splits = ppocr::conv_split_k(p);
   return name.c_str();
 }
 
@@ -615,7 +643,7 @@ int ppocr_probe_pair_bf16(const float* x, int m, int hw, int c, const float* gat
     q2.in = d_h, q2.C = q2.in_ps = 2 * c, q2.wt = d_w2, q2.ldw = 2 * c, q2.bias = static_cast<const float*>(d_b2);
     q2.Co = q2.out_ps = c, q2.out = d_o2;
     if (residual) q2.res = a, q2.res_ps = c;
-    if (ppocr::conv_split_k(m, 2 * c, c, BF) > 1 || ppocr::conv_split_k(m, c, 2 * c, BF) > 1) rc = 2;
+    if (ppocr::conv_split_k(q1) > 1 || ppocr::conv_split_k(q2) > 1) rc = 2;
     if (rc == 0) {
       ppocr::launch_conv(q1, nullptr);
       ppocr::launch_conv(q2, nullptr);

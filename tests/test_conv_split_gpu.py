@@ -1,0 +1,124 @@
+"""fp32 convolutions on the bf16 matrix cores (conv_split_kernel).
+
+Every fp32 operand is split into three bf16 parts and a product takes six of
+the nine partial products.  Each case asserts the kernel instance it runs and
+compares with a float64 convolution.  The bound per output is
+(K / 16 + 8) 2^-24 sum |a w| (the running fp32 sum is rounded once per 16
+products; the split itself and the terms left out are below 2^-24 of a
+product, and a gate product is rounded once), plus a few ulp of the output for
+the bias and the activation.
+"""
+import ctypes
+import zlib
+
+import numpy as np
+import pytest
+
+from test_conv_kernels_gpu import ACT_HSWISH, ACT_NONE, ACT_RELU, PROBE, _lib, _ptr, act, conv_ref
+
+# name, n, h, w, c, co, k, stride, pads (top, left, bottom, right), gated, splits, act, kernel
+CASES = [
+    ("1x1 whole tiles", 2, 64, 64, 64, 256, (1, 1), 1, (0, 0, 0, 0), False, 1, ACT_RELU, "conv_split<64x64,1x1>"),
+    ("1x1 M, N and K tails", 3, 61, 67, 100, 180, (1, 1), 1, (0, 0, 0, 0), False, 1, ACT_HSWISH,
+     "conv_split<64x64,1x1>"),
+    ("1x1 one column past a block", 1, 130, 131, 64, 68, (1, 1), 1, (0, 0, 0, 0), False, 1, ACT_NONE,
+     "conv_split<64x64,1x1>"),
+    ("1x1 even columns", 1, 130, 131, 72, 70, (1, 1), 1, (0, 0, 0, 0), False, 1, ACT_NONE, "conv_split<64x64,1x1>"),
+    ("gated, tiles straddling images", 9, 59, 41, 84, 132, (1, 1), 1, (0, 0, 0, 0), True, 1, ACT_RELU,
+     "conv_split<64x64,1x1,gate>"),
+    ("3x3 stride 1, channels not in 32", 1, 131, 127, 12, 128, (3, 3), 1, (1, 1, 1, 1), False, 1, ACT_RELU,
+     "conv_split<64x64>"),
+    ("3x3 stride 2", 2, 190, 200, 36, 160, (3, 3), 2, (1, 1, 1, 1), False, 1, ACT_HSWISH, "conv_split<64x64>"),
+    ("2x2 padded below", 1, 180, 190, 32, 64, (2, 2), 1, (0, 0, 1, 1), False, 1, ACT_RELU, "conv_split<64x64>"),
+    ("3x3 split K", 1, 127, 131, 128, 64, (3, 3), 1, (1, 1, 1, 1), False, 3, ACT_RELU, "conv_split<64x64>"),
+    ("1x1 split K, uneven", 1, 127, 131, 1060, 64, (1, 1), 1, (0, 0, 0, 0), False, 5, ACT_NONE,
+     "conv_split<64x64,1x1>"),
+    ("7x7 narrow", 2, 181, 190, 32, 32, (7, 7), 1, (3, 3, 3, 3), False, 1, ACT_NONE, "conv_split<128x32>"),
+    ("1x1 narrow, N tail", 1, 270, 256, 68, 28, (1, 1), 1, (0, 0, 0, 0), False, 1, ACT_RELU, "conv_split<128x32,1x1>"),
+    ("1x1 gated narrow", 3, 170, 140, 64, 24, (1, 1), 1, (0, 0, 0, 0), True, 1, ACT_RELU,
+     "conv_split<128x32,1x1,gate>"),
+    ("1x1 deep, wide tiles with tails", 2, 140, 141, 776, 772, (1, 1), 1, (0, 0, 0, 0), False, 1, ACT_RELU,
+     "conv_split<128x128,1x1>"),
+    ("3x3 deep, wide tiles", 2, 120, 129, 88, 516, (3, 3), 1, (1, 1, 1, 1), False, 1, ACT_NONE,
+     "conv_split<128x128>"),
+    ("fewer tiles stay on the fp32 kernel", 1, 40, 40, 64, 256, (1, 1), 1, (0, 0, 0, 0), False, 1, ACT_RELU,
+     "conv_gemm<64x32,1x1>"),
+]
+
+
+def _split_lib():
+    lib = _lib()
+    f, i = ctypes.POINTER(ctypes.c_float), ctypes.c_int
+    lib.ppocr_probe_conv_split3.argtypes = [f, i, i, i, i, f, f] + [i] * 10 + [f, i, f, ctypes.POINTER(i), f,
+                                                                               ctypes.POINTER(ctypes.c_char_p)]
+    lib.ppocr_probe_conv_split3.restype = i
+    return lib
+
+
+def _run(case, se=False):
+    name, n, h, w, c, co, (kh, kw), stride, pads, gated, splits, kind, want = case
+    rng = np.random.default_rng(zlib.crc32(name.encode()))
+    x = (rng.standard_normal((n, h, w, c)) * np.exp2(rng.integers(-6, 7, (n, h, w, c)))).astype(np.float32)
+    wt = (rng.standard_normal((co, c, kh, kw)) / np.sqrt(c * kh * kw)).astype(np.float32)
+    b = rng.standard_normal(co).astype(np.float32)
+    g = rng.uniform(0.0, 1.0, (n, c)).astype(np.float32) if gated else None
+    ho = (h + pads[0] + pads[2] - kh) // stride + 1
+    wo = (w + pads[1] + pads[3] - kw) // stride + 1
+    out = np.empty((n, ho, wo, co), dtype=np.float32)
+    kernel = ctypes.c_char_p()
+    rows = ctypes.c_int()
+    part = np.zeros((-(-ho * wo // 16) + 4, co), np.float32) if se else None
+    rc = _split_lib().ppocr_probe_conv_split3(_ptr(x), n, h, w, c, _ptr(wt), _ptr(b), co, kh, kw, stride, stride, *pads,
+                                              kind, _ptr(g), splits, _ptr(out), ctypes.byref(rows) if se else None,
+                                              _ptr(part), ctypes.byref(kernel))
+    assert rc == 0
+    assert kernel.value.decode() == want
+    xs = x.astype(np.float64) * (g[:, None, None, :] if gated else 1.0)
+    ref = conv_ref(xs, wt, b, (stride, stride), pads, ACT_NONE)
+    size = conv_ref(np.abs(xs), np.abs(wt), None, (stride, stride), pads, ACT_NONE)
+    tol = (c * kh * kw / 16 + 8) * 2.0 ** -24 * size + 2.0 ** -21 * np.abs(ref)
+    err = np.abs(out - act(ref, kind))
+    assert np.all(err <= tol), (name, float((err / tol).max()))
+    return out, part[:rows.value] if se else None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", CASES, ids=[c[0] for c in CASES])
+def test_split_conv_matches_float64(case):
+    _run(case)
+
+
+@pytest.mark.gpu
+def test_split_conv_leaves_se_sums():
+    """A single image's 1x1 layer also leaves its channel sums (two rows of
+    waves per 64-row tile), within fp32 summation order of the stored output."""
+    case = ("se sums", 1, 131, 129, 64, 132, (1, 1), 1, (0, 0, 0, 0), False, 1, ACT_RELU, "conv_split<64x64,1x1>")
+    out, part = _run(case, se=True)
+    assert part.shape[0] == -(-131 * 129 // 64) * 2
+    want = out.reshape(-1, out.shape[-1]).astype(np.float64)
+    assert np.all(np.abs(part.astype(np.float64).sum(0) - want.sum(0)) <= 1e-5 * np.abs(want).sum(0) + 1e-5)
+
+
+@pytest.mark.parametrize("co,k", [(32, 32), (33, 20), (70, 100)])
+def test_packed_parts_are_the_weights(co, k):
+    """The three parts of each weight add up to it within 2^-25, in the order
+    the 32x32x16 product reads: lane l of step s holds column l % 32 and
+    k = 16 s + 4 (l // 32) + i (i < 4) and 8 more from i = 4 on; zero past
+    the matrix (no GPU needed)."""
+    lib = ctypes.CDLL(str(PROBE))
+    lib.ppocr_probe_split3_size.restype = ctypes.c_size_t
+    rng = np.random.default_rng(co)
+    w = (rng.standard_normal((co, k)) * np.exp2(rng.integers(-20, 21, (co, k)))).astype(np.float32)
+    blocks, steps = -(-co // 32), 2 * -(-k // 32)
+    packed = np.empty((blocks, steps, 3, 64, 8), np.uint16)
+    assert lib.ppocr_probe_split3_size(co, k) == packed.size
+    lib.ppocr_probe_split3_weights(_ptr(w), co, k, packed.ctypes.data_as(ctypes.POINTER(ctypes.c_uint16)))
+    parts = (packed.astype(np.uint32) << 16).view(np.float32).astype(np.float64)
+    back = np.zeros((blocks * 32, steps * 16))
+    for lane in range(64):
+        for i in range(8):
+            at = 4 * (lane // 32) + i % 4 + 8 * (i // 4)
+            back[lane % 32::32, at::16] = parts[:, :, :, lane, i].sum(2)
+    assert np.all(np.abs(back[:co, :k] - w) <= 2.0 ** -25 * np.abs(w))
+    assert not back[co:].any() and not back[:, k:].any()
+    assert np.all(np.abs(parts[:, :, 1]) <= 2.0 ** -8 * np.abs(parts[:, :, 0]))
