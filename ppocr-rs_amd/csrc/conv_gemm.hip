@@ -1450,11 +1450,14 @@ __device__ __forceinline__ void lds_wait_to(floatx4& v) {
   asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(v) : "n"(N));
 }
 
+// S: stages of 32-deep slices.  KW = 2 (the 64x32 tile of small layers): each
+// block is shared by two waves, one per 16-deep step of a slice, whose sums
+// are added through LDS at the end, each wave finishing half of the rows.
 // PIPE: the second step's operands are read before the first step's MFMAs and
 // split beside them (the tiles that fit two workgroups per CU, where the other
 // workgroup's wave alone does not fill the matrix core: 1.10-1.25x there;
 // even on 64x64).
-template <int BM, int BN, int WM, int WN, bool PW, bool GATE, int EPI, bool PIPE>
+template <int BM, int BN, int WM, int WN, int KW, int S, bool PW, bool GATE, int EPI, bool PIPE>
 __device__ __forceinline__ void conv_split_tile(const ConvParams& p, int t) {
   constexpr int BK = 32;
   constexpr int TM = BM / (WM * 32), TN = BN / (WN * 32);
@@ -1463,16 +1466,20 @@ __device__ __forceinline__ void conv_split_tile(const ConvParams& p, int t) {
   constexpr int BP = (BKB + 3) / 4;              // per wave
   constexpr int STAGE = BM * 128 + BKB * 1024;
   constexpr int LDE = BN + 4;
-  static_assert(WM * WN == 4 && TM >= 1 && TN >= 1, "four waves of whole 32x32 blocks");
+  constexpr int EWM = WM * KW;                   // waves along the rows of the epilogue
+  static_assert(WM * WN * KW == 4 && TM >= 1 && TN >= 1, "four waves of whole 32x32 blocks");
+  static_assert(KW == 1 || (KW == 2 && WN == 1 && TM == 1 && TN == 1), "two waves share one block");
+  static_assert((S == 2 || S == 3) && (!PIPE || (S == 2 && KW == 1)), "stages");
   constexpr int STEP_READS = 2 * TM + 3 * TN;
   static_assert(STEP_READS <= 15, "LDS reads of a step fit the wait count");
-  constexpr int LDS = EPI == EPI_LDS && BM * LDE * 4 > 2 * STAGE ? BM * LDE * 4 : 2 * STAGE;
+  constexpr int LDS = EPI == EPI_LDS && BM * LDE * 4 > S * STAGE ? BM * LDE * 4 : S * STAGE;
   __shared__ __attribute__((aligned(1024))) char lds[LDS];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave / WN, wn = wave % WN;
+  const int kw = wave % KW;  // this wave's step of a slice (KW = 2)
+  const int wm = wave / KW / WN, wn = wave / KW % WN;
   const int lrow = lane & 31, half = lane >> 5;
   const int HoWo = p.Ho * p.Wo;
   const int M = p.N * HoWo;
@@ -1590,15 +1597,15 @@ __device__ __forceinline__ void conv_split_tile(const ConvParams& p, int t) {
   };
   // The gate values of a slice: [step][fragment half].
   struct Gates {
-    floatx4 v[GATE ? 2 : 1][2][TM];
+    floatx4 v[GATE ? 2 / KW : 1][2][TM];
   };
   auto load_gates = [&](int k0, Gates& gt) {
     if constexpr (GATE) {
 #pragma unroll
-      for (int kk = 0; kk < 2; ++kk)
+      for (int kk = 0; kk < 2 / KW; ++kk)
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
-          const int k = k0 + 16 * kk + 8 * q + 4 * half;
+          const int k = k0 + 16 * (KW == 2 ? kw : kk) + 8 * q + 4 * half;
 #pragma unroll
           for (int i = 0; i < TM; ++i)
             gt.v[kk][q][i] =
@@ -1689,10 +1696,10 @@ __device__ __forceinline__ void conv_split_tile(const ConvParams& p, int t) {
       __builtin_amdgcn_s_setprio(0);
     } else {
 #pragma unroll
-      for (int kk = 0; kk < 2; ++kk) {
+      for (int kk = 0; kk < 2 / KW; ++kk) {
         Step st;
         Split3 sp[TM];
-        read_step(stage, kk, st);
+        read_step(stage, KW == 2 ? kw : kk, st);
         wait_a(st, IB{});
         gate_step(gt, kk, st);
         split_step(st, sp);
@@ -1713,59 +1720,106 @@ __device__ __forceinline__ void conv_split_tile(const ConvParams& p, int t) {
       bias_pre[j] = make_float4(p.bias[bcol], p.bias[bcol + 1], 0.f, 0.f);
   }
 
-  // Slice s is in LDS once every wave has waited for its loads and passed
-  // the barrier, which also says that slice s - 1 is no longer read: its
-  // stage takes slice s + 1.
-  Gates g_cur{}, g_next{};
-  if (s_begin < s_end) {
-    issue(0, s_begin);
-    load_gates(s_begin * BK, g_next);
-  }
-  for (int s = s_begin; s < s_end; ++s) {
-    const int buf = (s - s_begin) & 1;
-    wait_vmcnt<0>();
-    stage_barrier();
-    if constexpr (GATE) g_cur = g_next;
-    if (s + 1 < s_end) {
-      issue(buf ^ 1, s + 1);
-      load_gates((s + 1) * BK, g_next);
+  // Slice s is in LDS once every wave has waited for its loads (the S - 2
+  // slices after it may still be loading) and passed the barrier, which also
+  // says that slice s - 1 is no longer read: its stage takes slice
+  // s + S - 1.  The gate values of a slice are loaded with it.
+  const int my_b = BKB % 4 == 0 ? BP : max(0, min(BP, BKB - wave * BP));
+  constexpr int G = GATE ? 4 / KW * TM : 0;
+  auto wait_slice = [&](bool last) {
+    if (S == 2 || last) {
+      wait_vmcnt<0>();
+    } else if (BKB % 4 == 0 || my_b == BP) {
+      wait_vmcnt<AP + BP + G>();
+    } else {
+      static_assert(BKB % 4 == 0 || BKB % BP == 0, "a wave has all its pieces or none");
+      wait_vmcnt<AP + G>();
     }
-    compute(buf, g_cur);
+  };
+  Gates gates[S];
+#pragma unroll
+  for (int i = 0; i < S - 1; ++i)
+    if (s_begin + i < s_end) {
+      issue(i, s_begin + i);
+      load_gates((s_begin + i) * BK, gates[i]);
+    }
+  auto step = [&](int buf, int refill, int s, const Gates& cur, Gates& next) {
+    wait_slice(s + 1 >= s_end);
+    stage_barrier();
+    if (s + S - 1 < s_end) {
+      issue(refill, s + S - 1);
+      load_gates((s + S - 1) * BK, next);
+    }
+    compute(buf, cur);
+  };
+  if constexpr (GATE) {
+    // Unrolled over the stages: the gate registers in flight stay in place.
+    for (int s = s_begin; s < s_end; s += S)
+#pragma unroll
+      for (int i = 0; i < S; ++i)
+        if (s + i < s_end) step(i, (i + S - 1) % S, s + i, gates[i], gates[(i + S - 1) % S]);
+  } else {
+    int buf = 0;
+    for (int s = s_begin; s < s_end; ++s) {
+      step(buf, buf == 0 ? S - 1 : buf - 1, s, gates[0], gates[0]);
+      buf = buf + 1 == S ? 0 : buf + 1;
+    }
   }
 
-  floatx4 out[4 * TM][TN];
+  floatx4 out[4 * TM / KW][TN];
+  if constexpr (KW == 2) {
+    // Wave kw keeps rows 16 kw .. + 15 of the block and takes the other wave's
+    // sums of them.
+    floatx4 give[2];
 #pragma unroll
-  for (int i = 0; i < TM; ++i)
+    for (int q = 0; q < 2; ++q)
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
+      for (int e = 0; e < 4; ++e) {
+        const float lo = acc[0][0][4 * q + e], hi = acc[0][0][8 + 4 * q + e];
+        out[q][0][e] = kw ? hi : lo;
+        give[q][e] = kw ? lo : hi;
+      }
+    __syncthreads();  // every wave is done with the stages
+    floatx4* swap = reinterpret_cast<floatx4*>(lds);
 #pragma unroll
-      for (int j = 0; j < TN; ++j)
-        out[4 * i + q][j] =
-            floatx4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+    for (int q = 0; q < 2; ++q) swap[(wave * 2 + q) * 64 + lane] = give[q];
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 2; ++q) out[q][0] += swap[((wave ^ 1) * 2 + q) * 64 + lane];
+  } else {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+          out[4 * i + q][j] =
+              floatx4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+  }
   if constexpr (EPI == EPI_DB) {
     static_assert(BM * (BN / 16) * 16 <= LDS, "DB partials fit the stages");
-    finish_db_regs<float, BM, BN, WM, WN, 32>(p, out, m0, n0, M, bias_pre, reinterpret_cast<float4*>(lds));
+    finish_db_regs<float, BM, BN, EWM, WN, 32>(p, out, m0, n0, M, bias_pre, reinterpret_cast<float4*>(lds));
   } else if constexpr (REGS) {
-    finish_regs<float, BM, BN, WM, WN, EPI == EPI_REGS_SE, 32>(p, out, m0, n0, M, bias_pre);
+    finish_regs<float, BM, BN, EWM, WN, EPI == EPI_REGS_SE, 32>(p, out, m0, n0, M, bias_pre);
   } else {
     __syncthreads();
     float* base = reinterpret_cast<float*>(lds);
-    finish_tile<float, BM, BN, WM, WN, 32>(
+    finish_tile<float, BM, BN, EWM, WN, 32>(
         p, out, [=](int row) { return base + row * LDE; }, m0, n0, M, n_tiles, &bias_pre[0]);
   }
 }
 
-template <int BM, int BN, int WM, int WN, bool PW, bool GATE, int EPI, bool PIPE>
+template <int BM, int BN, int WM, int WN, int KW, int S, bool PW, bool GATE, int EPI, bool PIPE>
 __global__ __launch_bounds__(256) void conv_split_kernel(ConvParams p) {
-  conv_split_tile<BM, BN, WM, WN, PW, GATE, EPI, PIPE>(p, xcd_tile());
+  conv_split_tile<BM, BN, WM, WN, KW, S, PW, GATE, EPI, PIPE>(p, xcd_tile());
 }
 
-template <int BM, int BN, int WM, int WN, bool PW, int EPI>
+template <int BM, int BN, int WM, int WN, int KW, int S, bool PW, int EPI>
 __global__ __launch_bounds__(256) void conv_split_multi_kernel(ConvMulti m) {
   int t = xcd_tile();
   int i = 0;
   while (i + 1 < m.count && t >= m.first[i + 1]) ++i;
-  conv_split_tile<BM, BN, WM, WN, PW, false, EPI, false>(m.p[i], t - m.first[i]);
+  conv_split_tile<BM, BN, WM, WN, KW, S, PW, false, EPI, false>(m.p[i], t - m.first[i]);
 }
 
 // ---------------------------------------------------------------------------
@@ -2297,22 +2351,24 @@ static void launch_tile_kernel(const ConvParams& p, dim3 grid, hipStream_t s) {
 }
 
 // Tile shapes of the split kernel (conv_split_tile).
-constexpr int kSplitBM[] = {64, 128, 128};
-constexpr int kSplitBN[] = {64, 128, 32};
-constexpr int kSplitWM[] = {2, 2, 4};
+constexpr int kSplitBM[] = {64, 128, 128, 64};
+constexpr int kSplitBN[] = {64, 128, 32, 32};
+constexpr int kSplitWM[] = {2, 2, 4, 2};
+constexpr int kSplitKW[] = {1, 1, 1, 2};
+constexpr int kSplitS[] = {2, 2, 2, 3};
 // The 128x128 tile reads ahead (PIPE) and finishes through LDS: its register
 // epilogue does not stay in registers.
-constexpr bool kSplitWide[] = {false, true, false};
+constexpr bool kSplitWide[] = {false, true, false, false};
 constexpr int kSplitMinTiles = 512;
-constexpr const char* kSplitName[] = {"64x64", "128x128", "128x32"};
+constexpr const char* kSplitName[] = {"64x64", "128x128", "128x32", "64x32"};
 
 // The split kernel's instance for a layer (split_tile).
 template <int I>
 static void launch_split_kernel(const ConvParams& p, dim3 grid, hipStream_t s) {
-  constexpr int BM = kSplitBM[I], BN = kSplitBN[I], WM = kSplitWM[I], WN = 4 / kSplitWM[I];
+  constexpr int BM = kSplitBM[I], BN = kSplitBN[I], WM = kSplitWM[I], KW = kSplitKW[I], WN = 4 / (WM * KW);
   const bool regs = regs_epilogue(p);
   auto go = [&](auto pw, auto gate, auto epi) {
-    hipLaunchKernelGGL((conv_split_kernel<BM, BN, WM, WN, decltype(pw)::value, decltype(gate)::value,
+    hipLaunchKernelGGL((conv_split_kernel<BM, BN, WM, WN, KW, kSplitS[I], decltype(pw)::value, decltype(gate)::value,
                                           decltype(epi)::value, kSplitWide[I]>),
                        grid, dim3(256), 0, s, p);
   };
@@ -2455,15 +2511,16 @@ static int pick_tile(int M, int cols, int dt) {
 }
 
 // The split kernel's tile for a layer, or -1 where the other kernels run it.
-// Measured against the fp32 kernels in the plans: from 512 tiles (two per CU)
-// 1.0-1.3x; below that the 64x32 fp32 tiles' shorter slices and larger number
-// of workgroups win (299-480 tiles without a split of K 0.7-0.95x, the
-// 40-pixel layers of one line 0.8-0.9x), except where K is deep enough to
-// split (K >= 1024 from 256 tiles: the one-page medium detector's head and
-// stem 3x3 convs 1.29x and 1.24x).  128x128 tiles take K >= 768 layers that
-// leave at least 900 of them (three and a half rounds of two per CU): 1.06-1.10x
-// against 64x64 at K = 768-1024, 0.96-0.99x at K = 512; not the gated
-// layers, whose gate values would cost the second workgroup of a CU, nor
+// Measured against the fp32 kernels in the plans: 64x64 (128x32 up to 32
+// columns) from 512 tiles, two per CU, 1.0-1.3x, and from 256 where K is deep
+// enough to split (K >= 1024: the one-page medium detector's head and stem
+// 3x3 convs 1.29x and 1.24x).  Below that the 64x32 tile, whose waves halve
+// the serial work of a slice: 1.1-1.35x at K >= 256, 1.0-1.16x on the 40- to
+// 480-pixel layers of one line; its gated or K < 256 layers of more than 600
+// tiles 0.84-0.97x, so they stay.  128x128 tiles take K >= 768 layers that
+// leave at least 900 of them (three and a half rounds of two per CU):
+// 1.06-1.10x against 64x64 at K = 768-1024, 0.96-0.99x at K = 512; not the
+// gated layers, whose gate values would cost the second workgroup of a CU, nor
 // those of one image, which may leave SE channel sums from registers.
 static int split_tile(const ConvParams& p) {
   if (!p.wt3 || p.dt != DT_F32) return -1;
@@ -2472,7 +2529,10 @@ static int split_tile(const ConvParams& p) {
     return (long)((M + kSplitBM[t] - 1) / kSplitBM[t]) * ((p.Co + kSplitBN[t] - 1) / kSplitBN[t]);
   };
   int t = p.Co <= 32 ? 2 : 0;
-  if (tiles(t) < kSplitMinTiles && !(K >= 1024 && tiles(t) >= kSplitMinTiles / 2)) return -1;
+  if (tiles(t) < kSplitMinTiles && !(K >= 1024 && tiles(t) >= kSplitMinTiles / 2)) {
+    if (p.db_ch || (K < 256 && tiles(3) >= 600)) return -1;
+    t = 3;
+  }
   if (K >= 768 && p.Co >= 128 && p.N > 1 && !p.in_gate && !p.db_ch && tiles(1) >= 900) t = 1;
   const int v = conv_variant(p, kSplitBM[t]);
   return v == CV_DIRECT_1X1 || v == CV_DIRECT || v == CV_DIRECT_GATE ? t : -1;
@@ -2512,7 +2572,7 @@ int conv_se_blocks(const ConvParams& p) {
   const int bm = tile_rows(p);
   if (conv_variant(p, bm) != CV_DIRECT_1X1) return 0;
   const int st = split_tile(p);
-  return (M + bm - 1) / bm * (st >= 0 ? kSplitWM[st] : kTileWM[pick_tile(M, p.Co, p.dt)]);
+  return (M + bm - 1) / bm * (st >= 0 ? kSplitWM[st] * kSplitKW[st] : kTileWM[pick_tile(M, p.Co, p.dt)]);
 }
 
 int conv_tile_cols(const ConvParams& p) { return tile_cols(p); }
@@ -2538,8 +2598,16 @@ int conv_split_k(const ConvParams& p) {
   if (Co % 4 != 0 || wide_shape(M, Co, K, dt)) return 1;
   long s;
   if (split_tile(p) >= 0) {
-    // Only the deep layers below kSplitMinTiles: three workgroups per CU.
-    return tiles < kSplitMinTiles ? (int)std::min<long>((768 + tiles - 1) / tiles, kMaxSplits) : 1;
+    if (split_tile(p) != 3)  // only the deep layers below kSplitMinTiles: three workgroups per CU
+      return tiles < kSplitMinTiles ? (int)std::min<long>((768 + tiles - 1) / tiles, kMaxSplits) : 1;
+    // 64x32 tiles leaving CUs idle, from 24 slices on (K = 512 1.0x, 896-1792
+    // 1.1-1.4x with at least eight slices a split), and from 12 where fewer
+    // than 64 tiles' loop is the whole time (1.25-1.4x with at least four).
+    const int nk = (K + 31) / 32;
+    const bool few = tiles < 64;
+    if (tiles >= 256 || nk < (few ? 12 : 24)) return 1;
+    s = std::min<long>({(512 + tiles - 1) / tiles, (long)nk / (few ? 4 : 8), (long)kMaxSplits});
+    return s >= 2 ? (int)s : 1;
   }
   const int bk = dt == DT_BF16 ? GemmTraits<bf16>::BK : GemmTraits<float>::BK;
   const int nk = (K + bk - 1) / bk;
@@ -2618,6 +2686,7 @@ static void launch_typed(const ConvParams& p, hipStream_t s) {
       case 0: launch_split_shape<0>(p, s); return;
       case 1: launch_split_shape<1>(p, s); return;
       case 2: launch_split_shape<2>(p, s); return;
+      case 3: launch_split_shape<3>(p, s); return;
       default: break;
     }
   }
@@ -2632,8 +2701,10 @@ static void launch_typed(const ConvParams& p, hipStream_t s) {
 }
 
 bool conv_takes_split3(int Co, int K) {
-  return Co >= 24 && K >= 64 && split3_size(Co, K) * 2 < kOutOfRange;
+  return Co >= 24 && K >= 48 && split3_size(Co, K) * 2 < kOutOfRange;
 }
+
+bool conv_runs_split(const ConvParams& p) { return split_tile(p) >= 0; }
 
 size_t split3_size(int Co, int K) {
   return (size_t)((Co + kSplitBlock - 1) / kSplitBlock) * ((K + 31) / 32) * (kSplitSlice / 2);
@@ -2735,10 +2806,10 @@ static void launch_multi_kernel(const ConvMulti& m, dim3 grid, hipStream_t s) {
 // Small layers share a launch, so never the 128x128 tile.
 template <int I>
 static void launch_split_multi(const ConvMulti& m, dim3 grid, hipStream_t s) {
-  constexpr int BM = kSplitBM[I], BN = kSplitBN[I], WM = kSplitWM[I], WN = 4 / kSplitWM[I];
+  constexpr int BM = kSplitBM[I], BN = kSplitBN[I], WM = kSplitWM[I], KW = kSplitKW[I], WN = 4 / (WM * KW);
   const ConvParams& p = m.p[0];
   auto go = [&](auto pw, auto epi) {
-    hipLaunchKernelGGL((conv_split_multi_kernel<BM, BN, WM, WN, decltype(pw)::value, decltype(epi)::value>), grid,
+    hipLaunchKernelGGL((conv_split_multi_kernel<BM, BN, WM, WN, KW, kSplitS[I], decltype(pw)::value, decltype(epi)::value>), grid,
                        dim3(256), 0, s, m);
   };
   using Lds = std::integral_constant<int, EPI_LDS>;
@@ -2765,6 +2836,7 @@ static void launch_multi_typed(const ConvMulti& m, dim3 grid, hipStream_t s) {
     switch (split_tile(m.p[0])) {
       case 0: launch_split_multi<0>(m, grid, s); return;
       case 2: launch_split_multi<2>(m, grid, s); return;
+      case 3: launch_split_multi<3>(m, grid, s); return;
       default: break;
     }
   }

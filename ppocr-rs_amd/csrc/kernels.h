@@ -252,7 +252,8 @@ std::string conv_kernel_name(const ConvParams& p);
 int conv_tile_cols(const ConvParams& p);
 // fp32 weights [Co][K] (K along a row) as the three-part bf16 operands of the
 // split conv kernel: split3_size() 16-bit values, zero past Co and K.
-bool conv_takes_split3(int Co, int K);  // layers the split kernel can run
+bool conv_takes_split3(int Co, int K);          // weights the split kernel can take
+bool conv_runs_split(const ConvParams& p);      // whether launch_conv runs the layer on it
 size_t split3_size(int Co, int K);
 void split3_weights(const float* w, int Co, int K, uint16_t* out);
 // Rows of the SE channel-sum array the conv leaves in se_part (single-image

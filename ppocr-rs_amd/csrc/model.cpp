@@ -305,8 +305,10 @@ class Builder {
   // where its kernel can (sp->P = 0 otherwise).  With `gated`, a bf16 layer
   // with an SE input gate returns there the x * g tensor its gate pass stores.
   // With `defer`, the op is returned there instead of added.
+  // `defer_split_k`: whether a deferred layer may split K (it then has its
+  // own launch).
   View conv(const View& x, const ConvW& w, const Epi& e, const std::string& name, SePartial* sp = nullptr,
-            View* gated = nullptr, Deferred* defer = nullptr) {
+            View* gated = nullptr, Deferred* defer = nullptr, bool defer_split_k = true) {
     if (x.c != w.ci_pad) raise(PPOCR_ERR_INVALID_MODEL, name + ": input has " + std::to_string(x.c) + " channels");
     const int Ho = (x.h + w.pt + w.pb - w.kh) / w.sh + 1;
     const int Wo = (x.w + w.pl + w.pr - w.kw) / w.sw + 1;
@@ -353,7 +355,7 @@ class Builder {
     base.dt = x.dt;
     size_t wo = w.w, bo = w.b, wo3 = w.w3;
     // Split-K workspace [splits][M][Co] fp32, live for this op only.
-    const int splits = conv_split_k(stand_in(base, a_src, w, has_ig && !prescale, 0));
+    const int splits = defer && !defer_split_k ? 1 : conv_split_k(stand_in(base, a_src, w, has_ig && !prescale, 0));
     View ws;
     if (splits > 1) ws = alloc(1, splits, x.n * Ho * Wo, w.co, name + ".split_k", DT_F32);
     base.splits = splits;
@@ -425,6 +427,20 @@ class Builder {
     return out;
   }
 
+  // Launch parameters of a plain layer as far as they choose its kernel.
+  static ConvParams shape_of(const View& x, const ConvW& w) {
+    ConvParams p{};
+    p.N = x.n, p.H = x.h, p.W = x.w, p.C = x.c, p.in_ps = x.ps;
+    p.Ho = (x.h + w.pt + w.pb - w.kh) / w.sh + 1;
+    p.Wo = (x.w + w.pl + w.pr - w.kw) / w.sw + 1;
+    p.Co = p.out_ps = w.co;
+    p.ldw = w.ldw;
+    p.kh = w.kh, p.kw = w.kw, p.sh = w.sh, p.sw = w.sw, p.pt = w.pt, p.pl = w.pl;
+    p.rep = 1;
+    p.dt = x.dt;
+    return stand_in(p, x, w, false, 0);
+  }
+
   // Independent conv layers (the levels of a neck), each set of them that
   // can share a launch (conv_multi_supported) as one op, the others one op
   // each; a set is named after `name` with its first layer's index.
@@ -434,8 +450,23 @@ class Builder {
     const int n = (int)xs.size();
     std::vector<View> outs(n);
     std::vector<Deferred> d(n);
-    for (int i = 0; i < n; ++i)
-      outs[i] = conv(*xs[i], ws[i], e, names[i], sps ? &(*sps)[i] : nullptr, nullptr, &d[i]);
+    // The levels run on one kind of kernel, the largest level's, so that they
+    // can share a launch: all on the split kernel, without splits of K (the
+    // small levels' workgroups fill in beside the large one's: the one-page
+    // medium detector's intraclass levels 78 launches for 90, 1.05x), or all
+    // on the fp32 kernels.
+    bool split3 = true;
+    size_t largest = 0;
+    for (int i = 0; i < n; ++i) {
+      split3 = split3 && ws[i].w3 != NOW;
+      if (xs[i]->pixels() > xs[largest]->pixels()) largest = i;
+    }
+    split3 = split3 && conv_runs_split(shape_of(*xs[largest], ws[largest]));
+    for (int i = 0; i < n; ++i) {
+      ConvW w = ws[i];
+      if (!split3) w.w3 = NOW;
+      outs[i] = conv(*xs[i], w, e, names[i], sps ? &(*sps)[i] : nullptr, nullptr, &d[i], !split3);
+    }
     // Greedy sets in layer order: a layer joins the first set it can share a
     // launch with.
     std::vector<std::vector<int>> sets;

@@ -41,8 +41,20 @@ CASES = [
      "conv_split<128x128,1x1>"),
     ("3x3 deep, wide tiles", 2, 120, 129, 88, 516, (3, 3), 1, (1, 1, 1, 1), False, 1, ACT_NONE,
      "conv_split<128x128>"),
-    ("fewer tiles stay on the fp32 kernel", 1, 40, 40, 64, 256, (1, 1), 1, (0, 0, 0, 0), False, 1, ACT_RELU,
-     "conv_gemm<64x32,1x1>"),
+    ("small 1x1 whole tiles", 1, 16, 24, 256, 64, (1, 1), 1, (0, 0, 0, 0), False, 1, ACT_RELU, "conv_split<64x32,1x1>"),
+    ("small 1x1 M, N and K tails", 2, 9, 13, 84, 46, (1, 1), 1, (0, 0, 0, 0), False, 1, ACT_HSWISH,
+     "conv_split<64x32,1x1>"),
+    ("small 1x1 one slice", 1, 5, 7, 48, 24, (1, 1), 1, (0, 0, 0, 0), False, 1, ACT_NONE, "conv_split<64x32,1x1>"),
+    ("small 1x1 two slices", 1, 5, 7, 64, 33, (1, 1), 1, (0, 0, 0, 0), False, 1, ACT_NONE, "conv_split<64x32,1x1>"),
+    ("small gated, many slices", 3, 9, 11, 420, 60, (1, 1), 1, (0, 0, 0, 0), True, 1, ACT_RELU,
+     "conv_split<64x32,1x1,gate>"),
+    ("small gated, one slice", 2, 8, 9, 52, 32, (1, 1), 1, (0, 0, 0, 0), True, 1, ACT_NONE,
+     "conv_split<64x32,1x1,gate>"),
+    ("small 3x3", 2, 13, 23, 20, 40, (3, 3), 1, (1, 1, 1, 1), False, 1, ACT_RELU, "conv_split<64x32>"),
+    ("small 3x3 stride 2, split K", 1, 26, 46, 64, 64, (3, 3), 2, (1, 1, 1, 1), False, 4, ACT_NONE,
+     "conv_split<64x32>"),
+    ("small 1x1 split K, uneven", 1, 13, 23, 900, 96, (1, 1), 1, (0, 0, 0, 0), False, 3, ACT_RELU,
+     "conv_split<64x32,1x1>"),
 ]
 
 
@@ -89,12 +101,15 @@ def test_split_conv_matches_float64(case):
 
 
 @pytest.mark.gpu
-def test_split_conv_leaves_se_sums():
-    """A single image's 1x1 layer also leaves its channel sums (two rows of
-    waves per 64-row tile), within fp32 summation order of the stored output."""
-    case = ("se sums", 1, 131, 129, 64, 132, (1, 1), 1, (0, 0, 0, 0), False, 1, ACT_RELU, "conv_split<64x64,1x1>")
+@pytest.mark.parametrize("h,w,co,waves,kernel", [(131, 129, 132, 2, "conv_split<64x64,1x1>"),
+                                                 (19, 23, 44, 4, "conv_split<64x32,1x1>")])
+def test_split_conv_leaves_se_sums(h, w, co, waves, kernel):
+    """A single image's 1x1 layer also leaves its channel sums (one row per
+    wave's rows of a 64-row tile), within fp32 summation order of the stored
+    output."""
+    case = ("se sums", 1, h, w, 64, co, (1, 1), 1, (0, 0, 0, 0), False, 1, ACT_RELU, kernel)
     out, part = _run(case, se=True)
-    assert part.shape[0] == -(-131 * 129 // 64) * 2
+    assert part.shape[0] == -(-h * w // 64) * waves
     want = out.reshape(-1, out.shape[-1]).astype(np.float64)
     assert np.all(np.abs(part.astype(np.float64).sum(0) - want.sum(0)) <= 1e-5 * np.abs(want).sum(0) + 1e-5)
 
