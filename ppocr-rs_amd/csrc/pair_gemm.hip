@@ -80,11 +80,52 @@ __device__ __forceinline__ void tile_product(const float* src, int lds, const fl
   }
 }
 
+// The weight vectors of KC slices from slice c0 on of a product of nk slices.
+__device__ __forceinline__ void load_chunk(float4 (&w)[KC], const float* wrow, int c0, int nk, int g) {
+#pragma unroll
+  for (int i = 0; i < KC; ++i)
+    if (c0 + i < nk) w[i] = *reinterpret_cast<const float4*>(wrow + (c0 + i) * 16 + 4 * g);
+}
+
+// NH 16-row tiles of src times 16 weight rows as tile_product (same sums),
+// with the first chunk of weights already in cur and the first chunk of the
+// wave's next product (next_row, next_nk slices; null: none) in it afterwards:
+// its loads are issued before this product's last slices.
+template <int NH>
+__device__ __forceinline__ void chained_product(const float* src, int lds, const float* wrow, int nk, int lrow, int g,
+                                                f32x4 (&acc)[NH], float4 (&cur)[KC], const float* next_row,
+                                                int next_nk) {
+#pragma unroll
+  for (int h = 0; h < NH; ++h) acc[h] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const float* ap = src + lrow * lds + 4 * g;
+  for (int c0 = 0; c0 < nk; c0 += KC) {
+    float4 nxt[KC];
+    if (c0 + KC < nk)
+      load_chunk(nxt, wrow, c0 + KC, nk, g);
+    else if (next_row)
+      load_chunk(nxt, next_row, 0, next_nk, g);
+#pragma unroll
+    for (int i = 0; i < KC; ++i)
+      if (c0 + i < nk)
+#pragma unroll
+        for (int h = 0; h < NH; ++h)
+          mfma4(acc[h], *reinterpret_cast<const float4*>(ap + h * 16 * lds + (c0 + i) * 16), cur[i]);
+#pragma unroll
+    for (int i = 0; i < KC; ++i) cur[i] = nxt[i];
+  }
+}
+
 // DW: the input tile is the 3x3 depthwise conv of p.dw_in at the tile's
 // pixels, summed as the depthwise kernels do (taps row-major, one fmaf per
 // tap and channel, zeros for taps in the padding, then the bias).
-template <bool GATE, bool RES, bool DW>
-__global__ __launch_bounds__(256) void pointwise_pair_kernel(PairParams p) {
+// NW waves.  A tile's time is a chain of latencies (input loads, the first
+// weights of each product, MFMAs of dependent accumulators): with eight waves
+// a wave has half the column tiles, each output tile's two row halves go to
+// two waves, the input tile loads in half the steps, and the weights of a
+// wave's next product load during the one before, the first ones beside the
+// input.  Sums and results are those of four waves.
+template <bool GATE, bool RES, bool DW, int NW>
+__global__ __launch_bounds__(64 * NW) void pointwise_pair_kernel(PairParams p) {
   extern __shared__ __attribute__((aligned(16))) float sm[];
   const int ldx = p.C + 4, ldh = p.H2 + 4;  // +4 floats: conflict-free 16-byte row reads
   float* xs = sm;                           // [PB_M][ldx]
@@ -93,6 +134,18 @@ __global__ __launch_bounds__(256) void pointwise_pair_kernel(PairParams p) {
   const int lane = tid & 63, wave = tid >> 6;
   const int lrow = lane & 15, g = lane >> 4;
   const int m0 = blockIdx.x * PB_M;
+
+  // Products of this wave: hidden column tiles wave, wave + NW, ..., then
+  // output units (column tile, and with eight waves a row half).
+  constexpr int NH = NW == 8 ? 1 : 2;  // row halves of an output unit
+  const int n_hid = p.H2 / 16, n_out = p.Co / 16 * (2 / NH);
+  auto hid_row = [&](int ct) { return p.w1 + (size_t)(ct * 16 + lrow) * p.ldw1; };
+  auto out_row = [&](int u) { return p.w2 + (size_t)(u / (2 / NH) * 16 + lrow) * p.ldw2; };
+  float4 wv[KC];
+  if (wave < n_hid)
+    load_chunk(wv, hid_row(wave), 0, p.C / 16, g);
+  else if (wave < n_out)
+    load_chunk(wv, out_row(wave), 0, p.H2 / 16, g);
 
   // SE gate formed here (GATE with se_part, one image): gs[c] in the hidden
   // tile's LDS, free until the hidden products.  Lane (ph, q) sums partial
@@ -169,7 +222,7 @@ __global__ __launch_bounds__(256) void pointwise_pair_kernel(PairParams p) {
 
   // Input tile, gated; rows past M are zero.
   const int c4 = p.C >> 2;
-  for (int i = tid; i < PB_M * c4; i += 256) {
+  for (int i = tid; i < PB_M * c4; i += 64 * NW) {
     const int r = i / c4, c = (i - r * c4) * 4;
     const int m = m0 + r;
     float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -211,34 +264,36 @@ __global__ __launch_bounds__(256) void pointwise_pair_kernel(PairParams p) {
 
   // Hidden tile: lane (lrow, g) of column tile ct holds rows 4g + v (and
   // 16 + 4g + v) of hidden channel ct * 16 + lrow.
-  for (int ct = wave; ct < p.H2 / 16; ct += 4) {
-    f32x4 acc0, acc1;
+  for (int ct = wave; ct < n_hid; ct += NW) {
+    f32x4 acc[2];
     const int col = ct * 16 + lrow;
-    tile_product(xs, ldx, p.w1 + (size_t)col * p.ldw1, p.C, lrow, g, acc0, acc1, p.C);
+    const bool more = ct + NW < n_hid;
+    const float* next = more ? hid_row(ct + NW) : wave < n_out ? out_row(wave) : nullptr;
     const float b = p.b1 ? p.b1[col] : 0.0f;
+    chained_product<2>(xs, ldx, hid_row(ct), p.C / 16, lrow, g, acc, wv, next, (more ? p.C : p.H2) / 16);
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      hs[(4 * g + v) * ldh + col] = act_apply(ACT_GELU, acc0[v] + b);
-      hs[(16 + 4 * g + v) * ldh + col] = act_apply(ACT_GELU, acc1[v] + b);
-    }
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) hs[(16 * h + 4 * g + v) * ldh + col] = act_apply(ACT_GELU, acc[h][v] + b);
   }
   __syncthreads();
 
   // Output tile.
-  for (int ct = wave; ct < p.Co / 16; ct += 4) {
-    f32x4 acc0, acc1;
+  for (int u = wave; u < n_out; u += NW) {
+    f32x4 acc[NH];
+    const int ct = u / (2 / NH), half0 = NH == 1 ? u & 1 : 0;
     const int col = ct * 16 + lrow;
-    tile_product(hs, ldh, p.w2 + (size_t)col * p.ldw2, p.H2, lrow, g, acc0, acc1, p.H2);
     const float b = p.b2 ? p.b2[col] : 0.0f;
+    chained_product<NH>(hs + half0 * 16 * ldh, ldh, out_row(u), p.H2 / 16, lrow, g, acc, wv,
+                        u + NW < n_out ? out_row(u + NW) : nullptr, p.H2 / 16);
 #pragma unroll
-    for (int half = 0; half < 2; ++half) {
-      const f32x4& acc = half ? acc1 : acc0;
+    for (int h = 0; h < NH; ++h) {
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        const int row = half * 16 + 4 * g + v;
+        const int row = (half0 + h) * 16 + 4 * g + v;
         const int m = m0 + row;
         if (m >= p.M) continue;
-        float o = acc[v] + b;
+        float o = acc[h][v] + b;
         if constexpr (RES) o = o + xs[row * ldx + col];  // the gated input, as the unfused residual
         p.out[(size_t)m * p.out_ps + col] = o;
       }
@@ -359,23 +414,38 @@ bool pair_se_fold_supported(int N, int C, int H2, int Cr, int P) {
 
 size_t pointwise_pair_lds(int C, int H2) { return (size_t)PB_M * ((C + 4) + (H2 + 4)) * sizeof(float); }
 
-void launch_pointwise_pair(const PairParams& p, hipStream_t s) {
-  const dim3 grid((unsigned)((p.M + PB_M - 1) / PB_M));
+template <int NW>
+static void launch_pair_waves(const PairParams& p, hipStream_t s) {
+  const dim3 grid((unsigned)((p.M + PB_M - 1) / PB_M)), block(64 * NW);
   const size_t lds = pointwise_pair_lds(p.C, p.H2);
   const bool gate = p.gate != nullptr || p.se_part != nullptr, res = p.residual != 0;
   if (p.dw_in) {
     if (res)
-      hipLaunchKernelGGL((pointwise_pair_kernel<false, true, true>), grid, dim3(256), lds, s, p);
+      hipLaunchKernelGGL((pointwise_pair_kernel<false, true, true, NW>), grid, block, lds, s, p);
     else
-      hipLaunchKernelGGL((pointwise_pair_kernel<false, false, true>), grid, dim3(256), lds, s, p);
+      hipLaunchKernelGGL((pointwise_pair_kernel<false, false, true, NW>), grid, block, lds, s, p);
   } else if (gate && res)
-    hipLaunchKernelGGL((pointwise_pair_kernel<true, true, false>), grid, dim3(256), lds, s, p);
+    hipLaunchKernelGGL((pointwise_pair_kernel<true, true, false, NW>), grid, block, lds, s, p);
   else if (gate)
-    hipLaunchKernelGGL((pointwise_pair_kernel<true, false, false>), grid, dim3(256), lds, s, p);
+    hipLaunchKernelGGL((pointwise_pair_kernel<true, false, false, NW>), grid, block, lds, s, p);
   else if (res)
-    hipLaunchKernelGGL((pointwise_pair_kernel<false, true, false>), grid, dim3(256), lds, s, p);
+    hipLaunchKernelGGL((pointwise_pair_kernel<false, true, false, NW>), grid, block, lds, s, p);
   else
-    hipLaunchKernelGGL((pointwise_pair_kernel<false, false, false>), grid, dim3(256), lds, s, p);
+    hipLaunchKernelGGL((pointwise_pair_kernel<false, false, false, NW>), grid, block, lds, s, p);
+}
+
+// Eight waves below 400 tiles, where the chain of one tile is the launch's
+// time (10-150 tiles 1.13-1.21x: tiny detector one page 12.5-15.7 -> 10.6-13.6
+// us a pair, 0.361 -> 0.341 ms in all); from there four, of which a CU holds
+// more beside each other (598 tiles 0.85x with eight, the batch-64 recognizer's
+// 960 and more 0.88-0.91x).
+constexpr int kPairFewTiles = 400;
+
+void launch_pointwise_pair(const PairParams& p, hipStream_t s) {
+  if ((p.M + PB_M - 1) / PB_M < kPairFewTiles)
+    launch_pair_waves<8>(p, s);
+  else
+    launch_pair_waves<4>(p, s);
 }
 
 }  // namespace ppocr
