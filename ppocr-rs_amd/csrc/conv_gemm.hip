@@ -2521,7 +2521,9 @@ static int pick_tile(int M, int cols, int dt) {
 // leave at least 900 of them (three and a half rounds of two per CU):
 // 1.06-1.10x against 64x64 at K = 768-1024, 0.96-0.99x at K = 512; not the
 // gated layers, whose gate values would cost the second workgroup of a CU, nor
-// those of one image, which may leave SE channel sums from registers.
+// those of one image, which may leave SE channel sums from registers.  A
+// 96-column layer would leave a quarter of its 64-column tiles empty (the
+// batch-64 tiny recognizer's K = 192 ones 0.89-0.93x).
 static int split_tile(const ConvParams& p) {
   if (!p.wt3 || p.dt != DT_F32) return -1;
   const int M = p.N * p.Ho * p.Wo, K = p.kh * p.kw * p.C;
@@ -2532,6 +2534,8 @@ static int split_tile(const ConvParams& p) {
   if (tiles(t) < kSplitMinTiles && !(K >= 1024 && tiles(t) >= kSplitMinTiles / 2)) {
     if (p.db_ch || (K < 256 && tiles(3) >= 600)) return -1;
     t = 3;
+  } else if (t == 0 && p.Co <= 96 && p.Co % 64 != 0 && p.Co % 64 <= 32 && K < 256) {
+    return -1;
   }
   if (K >= 768 && p.Co >= 128 && p.N > 1 && !p.in_gate && !p.db_ch && tiles(1) >= 900) t = 1;
   const int v = conv_variant(p, kSplitBM[t]);

@@ -123,7 +123,9 @@ __device__ __forceinline__ void chained_product(const float* src, int lds, const
 // a wave has half the column tiles, each output tile's two row halves go to
 // two waves, the input tile loads in half the steps, and the weights of a
 // wave's next product load during the one before, the first ones beside the
-// input.  Sums and results are those of four waves.
+// input.  Sums and results are those of four waves, which hold no weights
+// across the products (16-26 registers fewer: with 960 tiles the chained loads
+// took 1.09-1.13x as long).
 template <bool GATE, bool RES, bool DW, int NW>
 __global__ __launch_bounds__(64 * NW) void pointwise_pair_kernel(PairParams p) {
   extern __shared__ __attribute__((aligned(16))) float sm[];
@@ -135,17 +137,18 @@ __global__ __launch_bounds__(64 * NW) void pointwise_pair_kernel(PairParams p) {
   const int lrow = lane & 15, g = lane >> 4;
   const int m0 = blockIdx.x * PB_M;
 
-  // Products of this wave: hidden column tiles wave, wave + NW, ..., then
-  // output units (column tile, and with eight waves a row half).
-  constexpr int NH = NW == 8 ? 1 : 2;  // row halves of an output unit
-  const int n_hid = p.H2 / 16, n_out = p.Co / 16 * (2 / NH);
+  // With eight waves, this wave's products: hidden column tiles wave,
+  // wave + 8, ..., then output units (column tile, row half).
+  const int n_hid = p.H2 / 16, n_out = p.Co / 16 * 2;
   auto hid_row = [&](int ct) { return p.w1 + (size_t)(ct * 16 + lrow) * p.ldw1; };
-  auto out_row = [&](int u) { return p.w2 + (size_t)(u / (2 / NH) * 16 + lrow) * p.ldw2; };
+  auto out_row = [&](int u) { return p.w2 + (size_t)(u / 2 * 16 + lrow) * p.ldw2; };
   float4 wv[KC];
-  if (wave < n_hid)
-    load_chunk(wv, hid_row(wave), 0, p.C / 16, g);
-  else if (wave < n_out)
-    load_chunk(wv, out_row(wave), 0, p.H2 / 16, g);
+  if constexpr (NW == 8) {
+    if (wave < n_hid)
+      load_chunk(wv, hid_row(wave), 0, p.C / 16, g);
+    else if (wave < n_out)
+      load_chunk(wv, out_row(wave), 0, p.H2 / 16, g);
+  }
 
   // SE gate formed here (GATE with se_part, one image): gs[c] in the hidden
   // tile's LDS, free until the hidden products.  Lane (ph, q) sums partial
@@ -267,36 +270,52 @@ __global__ __launch_bounds__(64 * NW) void pointwise_pair_kernel(PairParams p) {
   for (int ct = wave; ct < n_hid; ct += NW) {
     f32x4 acc[2];
     const int col = ct * 16 + lrow;
-    const bool more = ct + NW < n_hid;
-    const float* next = more ? hid_row(ct + NW) : wave < n_out ? out_row(wave) : nullptr;
-    const float b = p.b1 ? p.b1[col] : 0.0f;
-    chained_product<2>(xs, ldx, hid_row(ct), p.C / 16, lrow, g, acc, wv, next, (more ? p.C : p.H2) / 16);
+    float b;
+    if constexpr (NW == 8) {
+      const bool more = ct + NW < n_hid;
+      const float* next = more ? hid_row(ct + NW) : wave < n_out ? out_row(wave) : nullptr;
+      b = p.b1 ? p.b1[col] : 0.0f;
+      chained_product<2>(xs, ldx, hid_row(ct), p.C / 16, lrow, g, acc, wv, next, (more ? p.C : p.H2) / 16);
+    } else {
+      tile_product(xs, ldx, hid_row(ct), p.C, lrow, g, acc[0], acc[1], p.C);
+      b = p.b1 ? p.b1[col] : 0.0f;
+    }
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) hs[(16 * h + 4 * g + v) * ldh + col] = act_apply(ACT_GELU, acc[h][v] + b);
+    for (int v = 0; v < 4; ++v) {
+      hs[(4 * g + v) * ldh + col] = act_apply(ACT_GELU, acc[0][v] + b);
+      hs[(16 + 4 * g + v) * ldh + col] = act_apply(ACT_GELU, acc[1][v] + b);
+    }
   }
   __syncthreads();
 
-  // Output tile.
-  for (int u = wave; u < n_out; u += NW) {
-    f32x4 acc[NH];
-    const int ct = u / (2 / NH), half0 = NH == 1 ? u & 1 : 0;
-    const int col = ct * 16 + lrow;
-    const float b = p.b2 ? p.b2[col] : 0.0f;
-    chained_product<NH>(hs + half0 * 16 * ldh, ldh, out_row(u), p.H2 / 16, lrow, g, acc, wv,
-                        u + NW < n_out ? out_row(u + NW) : nullptr, p.H2 / 16);
+  // Output rows row0 + v of column col.
+  auto store = [&](const f32x4& acc, int row0, int col, float b) {
 #pragma unroll
-    for (int h = 0; h < NH; ++h) {
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int row = (half0 + h) * 16 + 4 * g + v;
-        const int m = m0 + row;
-        if (m >= p.M) continue;
-        float o = acc[h][v] + b;
-        if constexpr (RES) o = o + xs[row * ldx + col];  // the gated input, as the unfused residual
-        p.out[(size_t)m * p.out_ps + col] = o;
-      }
+    for (int v = 0; v < 4; ++v) {
+      const int m = m0 + row0 + v;
+      if (m >= p.M) continue;
+      float o = acc[v] + b;
+      if constexpr (RES) o = o + xs[(row0 + v) * ldx + col];  // the gated input, as the unfused residual
+      p.out[(size_t)m * p.out_ps + col] = o;
+    }
+  };
+  if constexpr (NW == 8) {
+    for (int u = wave; u < n_out; u += NW) {
+      f32x4 acc[1];
+      const int col = u / 2 * 16 + lrow, row = (u & 1) * 16;
+      const float b = p.b2 ? p.b2[col] : 0.0f;
+      chained_product<1>(hs + row * ldh, ldh, out_row(u), p.H2 / 16, lrow, g, acc, wv,
+                         u + NW < n_out ? out_row(u + NW) : nullptr, p.H2 / 16);
+      store(acc[0], row + 4 * g, col, b);
+    }
+  } else {
+    for (int ct = wave; ct < p.Co / 16; ct += NW) {
+      f32x4 acc0, acc1;
+      const int col = ct * 16 + lrow;
+      tile_product(hs, ldh, p.w2 + (size_t)col * p.ldw2, p.H2, lrow, g, acc0, acc1, p.H2);
+      const float b = p.b2 ? p.b2[col] : 0.0f;
+      store(acc0, 4 * g, col, b);
+      store(acc1, 16 + 4 * g, col, b);
     }
   }
 }

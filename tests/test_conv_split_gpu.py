@@ -21,9 +21,9 @@ CASES = [
     ("1x1 whole tiles", 2, 64, 64, 64, 256, (1, 1), 1, (0, 0, 0, 0), False, 1, ACT_RELU, "conv_split<64x64,1x1>"),
     ("1x1 M, N and K tails", 3, 61, 67, 100, 180, (1, 1), 1, (0, 0, 0, 0), False, 1, ACT_HSWISH,
      "conv_split<64x64,1x1>"),
-    ("1x1 one column past a block", 1, 130, 131, 64, 68, (1, 1), 1, (0, 0, 0, 0), False, 1, ACT_NONE,
+    ("1x1 columns past a block", 1, 130, 131, 64, 132, (1, 1), 1, (0, 0, 0, 0), False, 1, ACT_NONE,
      "conv_split<64x64,1x1>"),
-    ("1x1 even columns", 1, 130, 131, 72, 70, (1, 1), 1, (0, 0, 0, 0), False, 1, ACT_NONE, "conv_split<64x64,1x1>"),
+    ("1x1 even columns", 1, 130, 131, 72, 134, (1, 1), 1, (0, 0, 0, 0), False, 1, ACT_NONE, "conv_split<64x64,1x1>"),
     ("gated, tiles straddling images", 9, 59, 41, 84, 132, (1, 1), 1, (0, 0, 0, 0), True, 1, ACT_RELU,
      "conv_split<64x64,1x1,gate>"),
     ("3x3 stride 1, channels not in 32", 1, 131, 127, 12, 128, (3, 3), 1, (1, 1, 1, 1), False, 1, ACT_RELU,
