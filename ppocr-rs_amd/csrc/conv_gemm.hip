@@ -14,7 +14,9 @@
 //     bf16: v_mfma_f32_16x16x32_bf16, one per tile per 32-deep K slice, fp32
 //     accumulation.
 //   * Each wave64 owns a TM x TN grid of 16x16 accumulators.
-//   * Most layers run conv_gemm_direct_kernel: operand rows are loaded
+//   * fp32 layers with enough tiles and depth run conv_split_kernel: operands
+//     split in three bf16 parts, six bf16 products per fp32 one (see there).
+//   * Most others run conv_gemm_direct_kernel: operand rows are loaded
 //     straight into LDS (buffer_load_dwordx4 ... lds) through a 3- or
 //     4-stage pipeline; fp32 1x1 layers with an SE input gate multiply the A
 //     fragments by gate rows staged in LDS.  The other gated layers (the gate

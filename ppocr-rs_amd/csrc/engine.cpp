@@ -99,7 +99,7 @@ struct PinnedStage {
     if (base) HIP_OK(hipHostFree(base));
     base = nullptr;
     bytes = used = 0;
-    HIP_OK(hipHostMalloc(reinterpret_cast<void**>(&base), n, hipHostMallocDefault));
+    HIP_OK(hipHostMalloc(reinterpret_cast<void**>(&base), n, hipHostMallocCoherent));
     bytes = n;
   }
 };

@@ -8,8 +8,9 @@
 // multiplied by the SE gate when the block has one, rounded to fp32 as the
 // unfused gather does; or, for blocks without SE, computed from the block
 // input by its 3x3 depthwise token conv, the reference's depthwise ->
-// pointwise strip fusion, src/cpu/backend.rs:697-816) are staged in LDS; the four waves compute the hidden
-// tile GELU(x W1^T + b1) on the matrix cores (v_mfma_f32_16x16x4f32), 16
+// pointwise strip fusion, src/cpu/backend.rs:697-816) are staged in LDS; the
+// four waves (eight in launches of few tiles) compute the hidden tile
+// GELU(x W1^T + b1) on the matrix cores (v_mfma_f32_16x16x4f32), 16
 // hidden channels at a time, into a second LDS tile; then the output tile
 // h W2^T + b2 (+ x for a residual block) from that, 16 output channels at a
 // time.  Weights stream from L2.  The sums run in the order of the unfused

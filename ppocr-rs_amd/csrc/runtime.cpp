@@ -44,17 +44,19 @@ struct DeviceBuffer {
 };
 
 // Pinned host area of a context, through which its synchronous calls exchange
-// data with the device (guarded by ctx->mu, idle between calls): small uploads
-// are copied in whole, downloads pass through kSlots slots.  Copies from and to
-// pageable memory block the host and go through the runtime's own staging:
-// 9.8 MB down 560 us plus 500 us for the finite check, 300 us through the
-// slots with the check in the same pass.
+// data with the device by copy kernels (guarded by ctx->mu, idle between
+// calls): inputs up to the slots' size are copied in whole, downloads pass
+// through the slots one piece each, and a further slot holds the tables and
+// records of the postprocess.  Copies from and to pageable memory block the
+// host and go through the runtime's own staging: 9.8 MB down 560 us plus
+// 500 us for the finite check, 300 us through the slots with the check in the
+// same pass.
 struct HostStage {
-  static constexpr size_t kSlots = 4, kSlot = (size_t)1 << 20;
+  static constexpr size_t kSlots = 4, kSlot = (size_t)1 << 20, kBytes = (kSlots + 1) * kSlot;
   char* base = nullptr;
   hipEvent_t done[kSlots] = {};
   void create() {
-    HIP_OK(hipHostMalloc(reinterpret_cast<void**>(&base), kSlots * kSlot, hipHostMallocDefault));
+    HIP_OK(hipHostMalloc(reinterpret_cast<void**>(&base), kBytes, hipHostMallocCoherent));
     for (hipEvent_t& e : done) HIP_OK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   }
   void destroy() {
@@ -288,21 +290,22 @@ struct DrainOnError {
   }
 };
 
-// Queues the upload of `bytes` of caller memory.  Up to half of the pinned
-// area they go through it, in pieces so that copying one overlaps the transfer
-// of the one before (nothing queued may still read the area: every call waits
-// for its results); more is as fast from pageable memory.
+// Queues the upload of `bytes` (a multiple of 4) of caller memory.  Up to the
+// size of the pinned slots they go through them, in pieces so that copying one
+// overlaps the transfer of the one before (nothing queued may still read the
+// area: every call waits for its results); more goes from pageable memory.
 void upload(ppocr_hip_ctx* ctx, void* dst, const void* src, size_t bytes) {
   constexpr size_t kPiece = HostStage::kSlot / 2;
-  if (bytes > HostStage::kSlots * HostStage::kSlot / 2) {
+  if (bytes > HostStage::kSlots * HostStage::kSlot) {
     HIP_OK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, ctx->stream));
     return;
   }
   for (size_t i = 0; i < bytes; i += kPiece) {
     const size_t n = std::min(kPiece, bytes - i);
     memcpy(ctx->stage.base + i, static_cast<const char*>(src) + i, n);
-    HIP_OK(hipMemcpyAsync(static_cast<char*>(dst) + i, ctx->stage.base + i, n, hipMemcpyHostToDevice, ctx->stream));
+    launch_host_copy(static_cast<char*>(dst) + i, ctx->stage.base + i, n, ctx->stream);
   }
+  HIP_OK(hipGetLastError());
 }
 
 // Copies the NCHW input items of chunk c into the staging buffer.
@@ -326,8 +329,9 @@ void check_output_cap(ppocr_hip_model* m, const float* out, size_t cap) {
 
 // Queues the download of chunk c's outputs into their place in `out` (pinned).
 void queue_download(ppocr_hip_model* m, float* out, size_t c) {
-  HIP_OK(hipMemcpyAsync(out + c * m->chunk * m->item_out, output_ptr(m), chunk_items(m, c) * m->item_out * sizeof(float),
-                        hipMemcpyDeviceToHost, m->ctx->stream));
+  launch_host_copy(out + c * m->chunk * m->item_out, output_ptr(m), chunk_items(m, c) * m->item_out * sizeof(float),
+                   m->ctx->stream);
+  HIP_OK(hipGetLastError());
 }
 
 // Downloads chunk c's outputs into their place in `out` through the pinned
@@ -338,16 +342,15 @@ void download_chunk(ppocr_hip_model* m, float* out, size_t c) {
   const size_t n = chunk_items(m, c) * m->item_out;
   float* dst = out + c * m->chunk * m->item_out;
   const float* src = output_ptr(m);
-  // Each transfer costs about 10 us whatever its size: one below 256 KB, two
-  // below 2 MB (1.1 MB in four pieces took 61 us, in one 29 us with nothing
-  // to overlap its copy), slots above.
+  // One piece below 256 KB, two below 2 MB, slots above.
   const size_t parts = n <= 65536 ? 1 : n <= 524288 ? 2 : 4;
-  const size_t piece = std::min(HostStage::kSlot / sizeof(float), (n + parts - 1) / parts);
+  const size_t piece = std::min(HostStage::kSlot / sizeof(float), ((n + parts - 1) / parts + 63) / 64 * 64);
   const size_t pieces = (n + piece - 1) / piece;
   auto slot = [&](size_t i) { return reinterpret_cast<float*>(ctx->stage.base + i % HostStage::kSlots * HostStage::kSlot); };
   auto len = [&](size_t i) { return std::min(piece, n - i * piece); };
   auto issue = [&](size_t i) {
-    HIP_OK(hipMemcpyAsync(slot(i), src + i * piece, len(i) * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
+    launch_host_copy(slot(i), src + i * piece, len(i) * sizeof(float), ctx->stream);
+    HIP_OK(hipGetLastError());
     HIP_OK(hipEventRecord(ctx->stage.done[i % HostStage::kSlots], ctx->stream));
   };
   for (size_t i = 0; i < std::min(pieces, HostStage::kSlots); ++i) issue(i);
@@ -616,14 +619,14 @@ void pack_geometry(char* dst, const float* corners, const int* content_w, size_t
   memcpy(dst + n * 8 * sizeof(float), content_w, n * sizeof(int));
 }
 
-// Queues the upload of items [first, first + n) of a packed geometry table
+// Queues the upload of items [first, first + n) of a packed (pinned) geometry table
 // of `total` items (corners, then widths) as an n-item table at `geo`.
 void upload_geometry_slice(ppocr_hip_ctx* ctx, const char* packet, size_t total, size_t first, size_t n) {
   char* geo = static_cast<char*>(ctx->geo);
-  HIP_OK(hipMemcpyAsync(geo, packet + first * 8 * sizeof(float), n * 8 * sizeof(float), hipMemcpyHostToDevice,
-                        ctx->stream));
-  HIP_OK(hipMemcpyAsync(geo + n * 8 * sizeof(float), packet + total * 8 * sizeof(float) + first * sizeof(int),
-                        n * sizeof(int), hipMemcpyHostToDevice, ctx->stream));
+  launch_host_copy(geo, packet + first * 8 * sizeof(float), n * 8 * sizeof(float), ctx->stream);
+  launch_host_copy(geo + n * 8 * sizeof(float), packet + total * 8 * sizeof(float) + first * sizeof(int),
+                   n * sizeof(int), ctx->stream);
+  HIP_OK(hipGetLastError());
 }
 
 // Sizes the context's device geometry buffer to at least `bytes`; a move
@@ -666,14 +669,14 @@ void preprocess_chunk(ppocr_hip_model* m, const ppocr_hip_image* image, const fl
   const bool direct = m->image_graph != nullptr;
   float* planes = direct ? nullptr : staging_ptr(m);
   void* nhwc4 = direct ? input_ptr(m) : nullptr;
-  if (packet_bytes(n) > (HostStage::kSlots - 1) * HostStage::kSlot) {
+  if (packet_bytes(n) > HostStage::kSlots * HostStage::kSlot) {
     run_preprocess(ctx, image, corners + first * 8, content_w + first, (int)n, (int)m->in_shape[3],
                    (int)m->in_shape[2], m->plan.detector, planes, nhwc4, m->plan.input.dt);
     return;
   }
   ensure_geometry(ctx, packet_bytes(n));
   pack_geometry(ctx->stage.base, corners + first * 8, content_w + first, n);
-  HIP_OK(hipMemcpyAsync(ctx->geo, ctx->stage.base, packet_bytes(n), hipMemcpyHostToDevice, ctx->stream));
+  launch_host_copy(ctx->geo, ctx->stage.base, packet_bytes(n), ctx->stream);
   enqueue_preprocess(ctx, image, ctx->geo, (int)n, (int)m->in_shape[3], (int)m->in_shape[2], m->plan.detector, planes,
                      nhwc4, m->plan.input.dt);
 }
@@ -1076,12 +1079,12 @@ std::vector<std::vector<HostDetection>> run_db(ppocr_hip_ctx* ctx, const float* 
     tables[4 * N + 2 * n] = (int)std::min<uint32_t>(t.content_width, INT32_MAX);
     tables[4 * N + 2 * n + 1] = (int)std::min<uint32_t>(t.content_height, INT32_MAX);
   }
-  // The tables and the results pass through the pinned area's last slot (an
-  // upload of the maps may still be reading the first half).
-  char* pinned = ctx->stage.base + (HostStage::kSlots - 1) * HostStage::kSlot;
+  // The tables and the results pass through the pinned area's further slot (an
+  // upload of the maps may still be reading the others).
+  char* pinned = ctx->stage.base + HostStage::kSlots * HostStage::kSlot;
   if (4 * tables.size() <= HostStage::kSlot) {
     memcpy(pinned, tables.data(), 4 * tables.size());
-    HIP_OK(hipMemcpyAsync(base + L.tables, pinned, 4 * tables.size(), hipMemcpyHostToDevice, ctx->stream));
+    launch_host_copy(base + L.tables, pinned, 4 * tables.size(), ctx->stream);
   } else {
     HIP_OK(hipMemcpyAsync(base + L.tables, tables.data(), 4 * tables.size(), hipMemcpyHostToDevice, ctx->stream));
   }
@@ -1119,8 +1122,9 @@ std::vector<std::vector<HostDetection>> run_db(ppocr_hip_ctx* ctx, const float* 
   std::vector<float> rec(12 * (size_t)first);
   constexpr size_t kRecAt = 256;
   static_assert(kRecAt + 12 * kDbFirstRecords * 4 <= HostStage::kSlot, "first records fit a slot");
-  HIP_OK(hipMemcpyAsync(pinned, p.counters, sizeof counters, hipMemcpyDeviceToHost, ctx->stream));
-  HIP_OK(hipMemcpyAsync(pinned + kRecAt, p.out, rec.size() * 4, hipMemcpyDeviceToHost, ctx->stream));
+  launch_host_copy(pinned, p.counters, sizeof counters, ctx->stream);
+  launch_host_copy(pinned + kRecAt, p.out, rec.size() * 4, ctx->stream);
+  HIP_OK(hipGetLastError());
   HIP_OK(hipStreamSynchronize(ctx->stream));
   memcpy(counters, pinned, sizeof counters);
   memcpy(rec.data(), pinned + kRecAt, rec.size() * 4);

@@ -84,3 +84,25 @@ def test_postprocess_buffer_is_shared_by_sizes(gpu):
                 assert a.score == b.score and np.array_equal(a.polygon, b.polygon)
         with pytest.raises(ppocr_hip.GpuError):
             gpu.db_postprocess(m, [(0, h, w, h)] * n)
+
+
+# Maps go up by copy kernels: 16-byte lanes where the size allows, else 4-byte
+# ones; whole and partial pieces of 2^17 values; 2^20 - 1 values, the most
+# below the pinned slots' 4 MiB that has a remainder, and more (no pinned
+# area).  A block of its own value at both ends of every map and of every
+# piece (scores are means of equal values: exact up to one rounding).
+@pytest.mark.parametrize("n,h,w", [(1, 33, 35), (3, 35, 61), (1, 256, 512), (1, 257, 511), (2, 701, 703),
+                                   (1, 1023, 1025), (1, 1024, 1024), (1, 1027, 1029)])
+def test_maps_arrive_whole(gpu, n, h, w):
+    m = np.zeros((n, h, w), np.float32)
+    rows = {0, h - 4} | {p // w for p in range(0, h * w, 1 << 17) if p // w < h - 12}  # blocks apart
+    want = [[] for _ in range(n)]
+    for i in range(n):
+        for k, r in enumerate(sorted(rows)):
+            for j, x in enumerate((0, w - 12)):
+                v = np.float32(0.6 + 0.005 * (2 * k + j) + 0.1 * i)
+                m[i, r:r + 4, x:x + 12] = v
+                want[i].append(float(v))
+    got = gpu.db_postprocess(m, [(w, h, w, h)] * n)
+    for g, v in zip(got, want):
+        assert np.allclose(sorted(d.score for d in g), sorted(v), atol=1e-6)
