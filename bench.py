@@ -98,33 +98,37 @@ def kernel_groups(stats):
     return groups
 
 
-def compute_peak(bound, precision="f32"):
-    """Peak TFLOP/s of a compute roof (matrix or vector)."""
+def compute_peak(bound, precision="f32", name=""):
+    """Peak TFLOP/s of a compute roof (matrix or vector).  The split kernels
+    compute an fp32 product as six bf16 ones, so a sixth of the bf16 peak is
+    their roof."""
     if bound == "mfma":
+        if name.startswith("conv_split"):
+            return PEAK_BF16_TFLOPS / 6
         return PEAK_BF16_TFLOPS if precision == "bf16" else PEAK_F32_TFLOPS
     return PEAK_VALU_F32_TFLOPS
 
 
-def bound_of(g, precision="f32"):
+def bound_of(g, precision="f32", name=""):
     """The roof a kernel group runs under (the roofline model): the compute
     roof its kernel is built for (matrix cores or vector ALUs) when its
     arithmetic intensity, algorithmic FLOPs per algorithmic HBM byte, reaches
     that roof's ridge point (peak FLOP/s over the 8 TB/s of HBM; 19.7 FLOP/B
-    for fp32 matrix products, 312.5 for bf16); below the ridge HBM is the
+    for fp32 matrix products, 52.1 for split ones, 312.5 for bf16); below the ridge HBM is the
     lower roof, and the group is measured against it (achieved bytes / 8 TB/s
     equals achieved FLOPs over the attainable intensity x bandwidth)."""
     if g["bound"] not in ("mfma", "valu") or g["bytes"] <= 0:
         return g["bound"]
-    ridge = compute_peak(g["bound"], precision) * 1e12 / (PEAK_HBM_GBS * 1e9)
+    ridge = compute_peak(g["bound"], precision, name) * 1e12 / (PEAK_HBM_GBS * 1e9)
     return g["bound"] if g["flops"] / g["bytes"] >= ridge else "hbm"
 
 
-def rate(g, precision="f32"):
+def rate(g, precision="f32", name=""):
     """(achieved, peak, unit) of a kernel group against its roof (bound_of)."""
     secs = g["ms"] * 1e-3
-    bound = bound_of(g, precision)
+    bound = bound_of(g, precision, name)
     if bound in ("mfma", "valu"):
-        return g["flops"] / secs / 1e12, compute_peak(bound, precision), "TFLOP/s"
+        return g["flops"] / secs / 1e12, compute_peak(bound, precision, name), "TFLOP/s"
     return g["bytes"] / secs / 1e9, PEAK_HBM_GBS, "GB/s"
 
 
@@ -134,8 +138,8 @@ def kernel_table(stats, top=12, precision="f32"):
     total_ms = sum(v["ms"] for v in groups.values())
     rows = []
     for name, g in sorted(groups.items(), key=lambda kv: -kv[1]["ms"])[:top]:
-        achieved, peak, unit = rate(g, precision)
-        rows.append({"kernel": name, "bound": bound_of(g, precision),
+        achieved, peak, unit = rate(g, precision, name)
+        rows.append({"kernel": name, "bound": bound_of(g, precision, name),
                      "launches_per_step": g["launches"], "ms_per_step": round(g["ms"], 4),
                      "share_of_device_time": round(g["ms"] / total_ms, 3) if total_ms else None,
                      "achieved": round(achieved, 2), "unit": unit, "frac": round(achieved / peak, 3)})
@@ -146,10 +150,10 @@ def roofline(stats, key, precision="f32"):
     """Dominant kernel instance: the one with the most device time per step."""
     groups = kernel_groups(stats)
     name, g = max(groups.items(), key=lambda kv: kv[1]["ms"])
-    achieved, peak, unit = rate(g, precision)
+    achieved, peak, unit = rate(g, precision, name)
     total_ms = sum(v["ms"] for v in groups.values())
     return {
-        "bound": bound_of(g, precision),
+        "bound": bound_of(g, precision, name),
         "achieved": round(achieved, 3),
         "peak": peak,
         "unit": unit,
