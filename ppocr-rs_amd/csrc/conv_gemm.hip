@@ -1377,12 +1377,16 @@ __global__ __launch_bounds__(256) void conv_gemm_direct_multi_kernel(ConvMulti m
 // l = bf16(x - h - m) (24 significant bits, both differences exact), and a
 // product takes the six partial products of weight down to 2^-16,
 // hh + hm + mh + hl + mm + lh, each exact and summed in the MFMA's fp32
-// accumulator: the three-way split of Henry, Tang and Heinecke (2019).  What
-// is left out is below 2^-25 of a product.  Against float64 the sums are
-// closer than the fp32 MFMA's: 2-norm error 1.7e-7, 2.1e-7, 3.0e-7 and 4.1e-7
-// at K = 128, 512, 1024 and 1792 where a chain of fp32 fused multiply-adds
-// leaves 2.1e-7, 3.8e-7, 5.8e-7 and 7.6e-7 (fewer roundings of the running
-// sum: one per 16 products instead of one per product).  Values that round to
+// accumulators: the three-way split of Henry, Tang and Heinecke (2019).  What
+// is left out (ml, lm and ll) is below 2^-24 of a product.  The hh products
+// have an accumulator of their own and the other five, whose sum is 2^-8 of
+// it, another, added once at the end, so the running sum is rounded once per
+// 16 products.  Measured against float64, the 2-norm error is 5.8e-8, 1.3e-7,
+// 1.9e-7 and 2.5e-7 at K = 96, 512, 1024 and 1792 where the fp32 kernel's
+// 16x16x4 MFMAs leave 1.8e-7, 4.1e-7, 5.7e-7 and 7.6e-7 (inputs of one sign:
+// 4.7e-8 to 2.0e-7 against 1.3e-7 to 5.4e-7).  With one accumulator for all
+// six it was 1.08-1.15 times the fp32 kernel's on inputs of one sign; the
+// second one costs 0.2-0.9 % of a plan's time.  Values that round to
 // infinity in bf16 (above 3.38e38) and infinities give NaN.
 //
 // What bounds it: six 32x32x16 MFMAs do the work of eight times as many fp32
@@ -1458,7 +1462,8 @@ __device__ __forceinline__ void lds_wait_to(floatx4& v) {
 // PIPE: the second step's operands are read before the first step's MFMAs and
 // split beside them (the tiles that fit two workgroups per CU, where the other
 // workgroup's wave alone does not fill the matrix core: 1.10-1.25x there;
-// even on 64x64).
+// even on 64x64).  Its 128 accumulator registers leave 128 for the rest at two
+// waves per SIMD, which it just fits without scratch.
 template <int BM, int BN, int WM, int WN, int KW, int S, bool PW, bool GATE, int EPI, bool PIPE>
 __device__ __forceinline__ void conv_split_tile(const ConvParams& p, int t) {
   constexpr int BK = 32;
@@ -1534,15 +1539,13 @@ __device__ __forceinline__ void conv_split_tile(const ConvParams& p, int t) {
       a_ix0[i] = ox * p.sw - p.pl;
     }
   }
-  // B: this wave fills pieces wave * BP .. + BP - 1 of the slice (block
-  // piece / 6), each lane its 16 bytes.
-  unsigned b_off[BP];
-#pragma unroll
-  for (int i = 0; i < BP; ++i) {
-    const int piece = wave * BP + i;
-    const int nb = n0 / kSplitBlock + piece / 6;
-    b_off[i] = nb < n_blocks ? (unsigned)nb * (unsigned)nk_all * kSplitSlice + (piece % 6) * 1024 + lane * 16 : kOutOfRange;
-  }
+  // B: this wave fills pieces wave * BP .. + BP - 1 of the slice, all of one
+  // block, each lane its 16 bytes.
+  static_assert(6 % BP == 0, "a wave's pieces are of one block");
+  const int b_block = n0 / kSplitBlock + wave * BP / 6;
+  const unsigned b_off = b_block < n_blocks
+                             ? (unsigned)b_block * (unsigned)nk_all * kSplitSlice + wave * BP % 6 * 1024 + lane * 16
+                             : kOutOfRange;
 
   const int s_begin = (int)((long)blockIdx.y * nk_all / gridDim.y);
   const int s_end = (int)((long)(blockIdx.y + 1) * nk_all / gridDim.y);
@@ -1573,7 +1576,7 @@ __device__ __forceinline__ void conv_split_tile(const ConvParams& p, int t) {
 #pragma unroll
     for (int i = 0; i < BP; ++i)
       if (BKB % 4 == 0 || wave * BP + i < BKB)
-        lds_load16(b_rsrc, b_off[i], (unsigned)s * kSplitSlice, stage + BM * 128 + (wave * BP + i) * 1024);
+        lds_load16(b_rsrc, b_off, (unsigned)s * kSplitSlice + i * 1024, stage + BM * 128 + (wave * BP + i) * 1024);
     if constexpr (!PW) {
       kc += BK;
       while (kc >= p.C) {
@@ -1586,13 +1589,14 @@ __device__ __forceinline__ void conv_split_tile(const ConvParams& p, int t) {
     }
   };
 
-  floatx16 acc[TM][TN];
+  // Sums of the hh products and of the five small ones.
+  floatx16 acc[TM][TN], low[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = low[i][j][e] = 0.f;
 
   struct Step {
     floatx4 a0[TM], a1[TM], b[TN][3];
@@ -1658,7 +1662,8 @@ __device__ __forceinline__ void conv_split_tile(const ConvParams& p, int t) {
         for (int i = 0; i < TM; ++i) {
           const u32x4 a = q == 0 ? sp[i].l : q == 2 || q == 3 ? sp[i].m : sp[i].h;
           const floatx4 b = q == 1 ? st.b[j][2] : q == 2 || q == 4 ? st.b[j][1] : st.b[j][0];
-          acc[i][j] = mfma_32x32(a, b, acc[i][j]);
+          floatx16& sum = q < 5 ? low[i][j] : acc[i][j];
+          sum = mfma_32x32(a, b, sum);
         }
   };
   auto wait_a = [&](Step& st, auto left) {
@@ -1713,9 +1718,9 @@ __device__ __forceinline__ void conv_split_tile(const ConvParams& p, int t) {
 
   constexpr bool REGS = EPI != EPI_LDS;
   constexpr int NB = REGS ? TN : 1;
-  float4 bias_pre[NB];
+  float4 bias_pre[NB];  // not with PIPE, which has no registers to spare
 #pragma unroll
-  for (int j = 0; j < NB; ++j) {
+  for (int j = 0; j < (PIPE ? 0 : NB); ++j) {
     const int bcol = REGS ? regs_col<BN, WN, 32>(n0, j) : staged_col<BN>(n0);
     bias_pre[j] = p.splits > 1 ? float4{0.f, 0.f, 0.f, 0.f} : bias4(p, bcol);
     if (REGS && p.splits <= 1 && p.bias && bcol + 1 < p.Co && bcol + 3 >= p.Co)
@@ -1768,6 +1773,10 @@ __device__ __forceinline__ void conv_split_tile(const ConvParams& p, int t) {
     }
   }
 
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] += low[i][j];
   floatx4 out[4 * TM / KW][TN];
   if constexpr (KW == 2) {
     // Wave kw keeps rows 16 kw .. + 15 of the block and takes the other wave's
@@ -1807,12 +1816,12 @@ __device__ __forceinline__ void conv_split_tile(const ConvParams& p, int t) {
     __syncthreads();
     float* base = reinterpret_cast<float*>(lds);
     finish_tile<float, BM, BN, EWM, WN, 32>(
-        p, out, [=](int row) { return base + row * LDE; }, m0, n0, M, n_tiles, &bias_pre[0]);
+        p, out, [=](int row) { return base + row * LDE; }, m0, n0, M, n_tiles, PIPE ? nullptr : &bias_pre[0]);
   }
 }
 
 template <int BM, int BN, int WM, int WN, int KW, int S, bool PW, bool GATE, int EPI, bool PIPE>
-__global__ __launch_bounds__(256) void conv_split_kernel(ConvParams p) {
+__global__ __launch_bounds__(256, PIPE ? 2 : 1) void conv_split_kernel(ConvParams p) {
   conv_split_tile<BM, BN, WM, WN, KW, S, PW, GATE, EPI, PIPE>(p, xcd_tile());
 }
 

@@ -114,6 +114,38 @@ def test_split_conv_leaves_se_sums(h, w, co, waves, kernel):
     assert np.all(np.abs(part.astype(np.float64).sum(0) - want.sum(0)) <= 1e-5 * np.abs(want).sum(0) + 1e-5)
 
 
+# Inputs of one sign (as after a ReLU) let the running sum grow with every
+# product, where each of its roundings counts most.
+@pytest.mark.gpu
+@pytest.mark.parametrize("positive", [True, False])
+@pytest.mark.parametrize("h,w,k,co,kernel", [(64, 128, 96, 256, "conv_split<64x64,1x1>"),
+                                             (64, 128, 512, 256, "conv_split<64x64,1x1>"),
+                                             (256, 260, 192, 32, "conv_split<128x32,1x1>"),
+                                             (8, 16, 96, 256, "conv_split<64x32,1x1>"),
+                                             (8, 16, 1024, 256, "conv_split<64x32,1x1>"),
+                                             (128, 130, 800, 512, "conv_split<128x128,1x1>")])
+def test_split_conv_is_as_accurate_as_fp32(h, w, k, co, kernel, positive):
+    """The 2-norm error against float64 is not above the fp32 matrix
+    instructions' on the same layer, for inputs of both signs and of one."""
+    lib = _split_lib()
+    n = 2 if "128x128" in kernel else 1
+    rng = np.random.default_rng(k + co)
+    x = rng.standard_normal((n, h, w, k)).astype(np.float32)
+    if positive:
+        x = np.maximum(x, 0)
+    wt = (rng.standard_normal((co, k, 1, 1)) / np.sqrt(k)).astype(np.float32)
+    one = [co, 1, 1, 1, 1, 0, 0, 0, 0, ACT_NONE, None, 1]
+    plain, split = (np.empty((n, h, w, co), np.float32) for _ in range(2))
+    assert lib.ppocr_probe_conv(_ptr(x), n, h, w, k, _ptr(wt), None, *one, 0, _ptr(plain)) == 0
+    name = ctypes.c_char_p()
+    assert lib.ppocr_probe_conv_split3(_ptr(x), n, h, w, k, _ptr(wt), None, *one, _ptr(split), None, None,
+                                       ctypes.byref(name)) == 0
+    assert name.value.decode() == kernel
+    ref = (x.reshape(-1, k).astype(np.float64) @ wt[:, :, 0, 0].T.astype(np.float64)).reshape(plain.shape)
+    err = [np.linalg.norm(o - ref) / np.linalg.norm(ref) for o in (split, plain)]
+    assert err[0] <= err[1], err
+
+
 @pytest.mark.parametrize("co,k", [(32, 32), (33, 20), (70, 100)])
 def test_packed_parts_are_the_weights(co, k):
     """The three parts of each weight add up to it within 2^-25, in the order
