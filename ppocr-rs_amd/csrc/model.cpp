@@ -1810,7 +1810,10 @@ void plan_arena(Plan& plan) {
   for (auto& b : plan.bufs) {
     if (b.first < 0) b.first = b.last = 0;
   }
+  // The input is written before a pass and kept through it: benchmark and
+  // profile run the plan again on the same input.
   plan.bufs[plan.staging].first = 0;
+  plan.bufs[plan.staging].last = end;
   plan.bufs[plan.output].last = end;
   std::vector<int> order(plan.bufs.size());
   for (size_t i = 0; i < order.size(); ++i) order[i] = (int)i;

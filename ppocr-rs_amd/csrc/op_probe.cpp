@@ -782,4 +782,36 @@ long ppocr_probe_plan_rounding(const char* path, int kind, int size, int n, int 
   }
 }
 
+// A model's plan, built on the host from a safetensors file (no device work),
+// as lines "<op>\t<kernel>", then "input kept" unless another buffer shares
+// arena bytes with the input, and "weights <bytes>".  Arguments and result as
+// ppocr_probe_plan_rounding; greedy: the recognizer's decoded form.
+long ppocr_probe_plan(const char* path, int kind, int size, int n, int h, int w, int dt, int greedy, char* out,
+                      size_t cap) {
+  try {
+    ppocr::SafeTensors st = ppocr::SafeTensors::load(path);
+    const size_t nchw[4] = {(size_t)n, 3, (size_t)h, (size_t)w};
+    ppocr::Plan plan = kind == 0 ? ppocr::build_detector(st, size, nchw, dt)
+                                 : ppocr::build_recognizer(st, size, nchw, dt, greedy != 0);
+    std::string text;
+    for (const ppocr::Op& op : plan.ops) text += op.name + "\t" + op.kernel + "\n";
+    const ppocr::Buffer& input = plan.bufs[plan.staging];
+    bool kept = true;
+    for (const ppocr::Buffer& b : plan.bufs)
+      if (&b != &input && b.bytes && b.arena_off < input.arena_off + input.bytes &&
+          input.arena_off < b.arena_off + b.bytes)
+        kept = false;
+    if (kept) text += "input kept\n";
+    text += "weights " + std::to_string(plan.weights.size()) + "\n";
+    if (out && cap) {
+      const size_t k = std::min(cap - 1, text.size());
+      memcpy(out, text.data(), k);
+      out[k] = 0;
+    }
+    return (long)text.size() + 1;
+  } catch (...) {
+    return -1;
+  }
+}
+
 }  // extern "C"
