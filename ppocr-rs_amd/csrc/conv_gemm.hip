@@ -1386,8 +1386,10 @@ __global__ __launch_bounds__(256) void conv_gemm_direct_multi_kernel(ConvMulti m
 // 16x16x4 MFMAs leave 1.8e-7, 4.1e-7, 5.7e-7 and 7.6e-7 (inputs of one sign:
 // 4.7e-8 to 2.0e-7 against 1.3e-7 to 5.4e-7).  With one accumulator for all
 // six it was 1.08-1.15 times the fp32 kernel's on inputs of one sign; the
-// second one costs 0.2-0.9 % of a plan's time.  Values that round to
-// infinity in bf16 (above 3.38e38) and infinities give NaN.
+// second one costs 0.2-0.9 % of a plan's time.  Outputs that parts beyond
+// bf16's range would turn into NaN are formed again in fp32 (fp32_element);
+// below 2^-110 a value's low parts reach bf16's smallest, 2^-133, and it is
+// off by up to half of that.
 //
 // What bounds it: six 32x32x16 MFMAs do the work of eight times as many fp32
 // ones' cycles (2.5 / 6 = 0.42 PFLOP/s against 0.157), and on dense random
@@ -1454,6 +1456,34 @@ __device__ __forceinline__ floatx4 lds_read16_at(unsigned addr) {
 template <int N>
 __device__ __forceinline__ void lds_wait_to(floatx4& v) {
   asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(v) : "n"(N));
+}
+
+// Element (m, n) over k values k0 .. k1 - 1 as a chain of fp32 fused
+// multiply-adds, up to the first NaN.
+template <bool PW, bool GATE>
+__device__ __forceinline__ float fp32_element(const ConvParams& p, int m, int n, int k0, int k1) {
+  const float* w = static_cast<const float*>(p.wt) + (size_t)n * p.ldw;
+  const float* x = static_cast<const float*>(p.in);
+  const int img = m / (p.Ho * p.Wo);
+  const int rem = m - img * (p.Ho * p.Wo);
+  const int oy = rem / p.Wo;
+  const int iy0 = oy * p.sh - p.pt, ix0 = (rem - oy * p.Wo) * p.sw - p.pl;
+  float sum = 0.f;
+#pragma unroll 1
+  for (int k = k0; k < k1 && sum == sum; ++k) {
+    float v = 0.f;
+    if constexpr (PW) {
+      v = x[(size_t)m * p.in_ps + k];
+    } else {
+      const int tap = k / p.C, ky = tap / p.kw;
+      const int iy = iy0 + ky, ix = ix0 + tap - ky * p.kw;
+      if ((unsigned)iy < (unsigned)p.H && (unsigned)ix < (unsigned)p.W)
+        v = x[((size_t)(img * p.H + iy) * p.W + ix) * p.in_ps + (k - tap * p.C)];
+    }
+    if constexpr (GATE) v = mul_rn(v, p.in_gate[(size_t)img * p.C + k]);
+    sum = fmaf(v, w[k], sum);
+  }
+  return sum;
 }
 
 // S: stages of 32-deep slices.  KW = 2 (the 64x32 tile of small layers): each
@@ -1777,7 +1807,8 @@ __device__ __forceinline__ void conv_split_tile(const ConvParams& p, int t) {
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j) acc[i][j] += low[i][j];
-  floatx4 out[4 * TM / KW][TN];
+  constexpr int OM = 4 * TM / KW;  // groups of eight rows a wave finishes
+  floatx4 out[OM][TN];
   if constexpr (KW == 2) {
     // Wave kw keeps rows 16 kw .. + 15 of the block and takes the other wave's
     // sums of them.
@@ -1806,6 +1837,31 @@ __device__ __forceinline__ void conv_split_tile(const ConvParams& p, int t) {
         for (int j = 0; j < TN; ++j)
           out[4 * i + q][j] =
               floatx4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+  }
+  // A value that is infinite, or above 3.38e38 and so infinite in bf16, splits
+  // into parts that add up to NaN, as do products beyond the fp32 range: what
+  // did not come out finite is formed again in fp32 (a finite total says that
+  // every value is; one vector add per value).
+  float total = 0.f;
+#pragma unroll
+  for (int i = 0; i < OM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) total += (out[i][j][0] + out[i][j][1]) + (out[i][j][2] + out[i][j][3]);
+  if (__builtin_expect(__any(!__builtin_isfinite(total)), 0)) {
+    const int row = m0 + wave / WN * OM * 8 + half * 4, col = n0 + wn * TN * 32 + lrow;
+#pragma unroll 1
+    for (int q = 0; q < OM * TN * 4; ++q) {
+      const int m = row + q / (TN * 4) * 8 + q % 4, n = col + q / 4 % TN * 32;
+      float v = 0.f;
+#pragma unroll
+      for (int r = 0; r < OM * TN * 4; ++r)
+        if (r == q) v = out[r / (TN * 4)][r / 4 % TN][r % 4];
+      if (!__builtin_isfinite(v) && m < M && n < p.Co)
+        v = fp32_element<PW, GATE>(p, m, n, s_begin * BK, min(s_end * BK, K));
+#pragma unroll
+      for (int r = 0; r < OM * TN * 4; ++r)
+        if (r == q) out[r / (TN * 4)][r / 4 % TN][r % 4] = v;
+    }
   }
   if constexpr (EPI == EPI_DB) {
     static_assert(BM * (BN / 16) * 16 <= LDS, "DB partials fit the stages");

@@ -146,6 +146,91 @@ def test_split_conv_is_as_accurate_as_fp32(h, w, k, co, kernel, positive):
     assert err[0] <= err[1], err
 
 
+def _probe(x, wt, stride, pads, gate, splits, kind):
+    """Output and kernel name of one layer on the split path, without bias."""
+    n, h, w, c = x.shape
+    co, _, kh, kw = wt.shape
+    ho, wo = (h + pads[0] + pads[2] - kh) // stride + 1, (w + pads[1] + pads[3] - kw) // stride + 1
+    out = np.empty((n, ho, wo, co), np.float32)
+    name = ctypes.c_char_p()
+    assert _split_lib().ppocr_probe_conv_split3(_ptr(x), n, h, w, c, _ptr(wt), None, co, kh, kw, stride, stride, *pads,
+                                                kind, _ptr(gate), splits, _ptr(out), None, None,
+                                                ctypes.byref(name)) == 0
+    return out, name.value.decode()
+
+
+# name, n, h, w, c, co, k, pads, gated, splits, kernel
+RANGE_CASES = [
+    ("64x64", 1, 128, 130, 64, 132, (1, 1), (0, 0, 0, 0), False, 1, "conv_split<64x64,1x1>"),
+    ("64x64 gated", 2, 96, 90, 68, 128, (1, 1), (0, 0, 0, 0), True, 1, "conv_split<64x64,1x1,gate>"),
+    ("64x64 3x3 split K", 1, 127, 131, 128, 64, (3, 3), (1, 1, 1, 1), False, 3, "conv_split<64x64>"),
+    ("128x32 odd columns", 1, 270, 256, 68, 27, (1, 1), (0, 0, 0, 0), False, 1, "conv_split<128x32,1x1>"),
+    ("128x128", 2, 120, 129, 88, 516, (3, 3), (1, 1, 1, 1), False, 1, "conv_split<128x128>"),
+    ("64x32", 1, 20, 30, 84, 46, (1, 1), (0, 0, 0, 0), False, 1, "conv_split<64x32,1x1>"),
+    ("64x32 gated split K", 3, 9, 11, 900, 60, (1, 1), (0, 0, 0, 0), True, 3, "conv_split<64x32,1x1,gate>"),
+]
+
+
+# A bf16 part of an infinite value, or of one above 3.38e38, is infinite.
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", RANGE_CASES, ids=[c[0] for c in RANGE_CASES])
+def test_infinities_and_the_top_of_the_range(case):
+    """Infinite inputs and weights give infinities and NaN as the products of
+    real numbers do, finite values of any size finite results, and other
+    outputs are untouched."""
+    name, n, h, w, c, co, (kh, kw), pads, gated, splits, want = case
+    rng = np.random.default_rng(zlib.crc32(name.encode()))
+    x = rng.standard_normal((n, h, w, c)).astype(np.float32)
+    wt = (rng.standard_normal((co, c, kh, kw)) / np.sqrt(c * kh * kw)).astype(np.float32)
+    wt[np.abs(wt) < 1e-6] = 1e-3
+    gate = rng.uniform(0.1, 1.0, (n, c)).astype(np.float32) if gated else None
+    x[..., c // 2] *= 0.01  # meets a weight of 3.395e38 below
+    top = np.finfo(np.float32).max
+    for at, v in [((0, 0, 0, 0), np.inf), ((0, 3, 5, 7), -np.inf), ((n - 1, h - 1, w - 1, c - 1), top),
+                  ((n - 1, h // 2, 2, c // 2), -top), ((0, h // 2, w // 2, 1), np.float32(3.39e38)),
+                  ((0, h - 2, 1, 33), np.nan)]:
+        x[at] = v
+    wt[3, c // 2, 0, 0] = np.float32(3.395e38)
+    wt[co - 1, 0, 0, 0] = np.inf
+    out, kernel = _probe(x, wt, 1, pads, gate, splits, ACT_NONE)
+    assert kernel == want
+    with np.errstate(invalid="ignore", over="ignore"):
+        xs = x.astype(np.float64) * (gate[:, None, None, :] if gated else 1.0)
+        ref = conv_ref(xs, wt, None, (1, 1), pads, ACT_NONE)
+        size = conv_ref(np.abs(xs), np.abs(wt), None, (1, 1), pads, ACT_NONE)
+        near = size > 2.0 ** 127  # may overflow on the way
+        wide = ref.astype(np.float32)
+        assert np.isinf(wide[~near]).sum() == 0
+        special = ~np.isfinite(ref)
+        assert np.array_equal(out[special], ref[special].astype(np.float32), equal_nan=True)
+        assert np.isinf(out[special]).any() and np.isnan(out[special]).any()
+        plain = ~near & ~special
+        k = c * kh * kw
+        assert np.all(np.abs(out - ref)[plain] <= ((k + 8) * 2.0 ** -24 * size)[plain])
+        assert np.abs(ref[plain]).max() > 1e36
+        relu, _ = _probe(x, wt, 1, pads, gate, splits, ACT_RELU)
+        assert np.array_equal(relu[~near], np.fmax(out, 0.0)[~near])
+        assert np.array_equal(relu[np.isposinf(ref)], np.full(np.isposinf(ref).sum(), np.inf, np.float32))
+
+
+# The low parts of a value below 2^-110 reach bf16's smallest, 2^-133.
+@pytest.mark.gpu
+@pytest.mark.parametrize("scale", [2.0 ** -100, 2.0 ** -112, 2.0 ** -120, 2.0 ** -126])
+@pytest.mark.parametrize("small_weights", [False, True])
+def test_the_bottom_of_the_range(scale, small_weights):
+    """Denormal parts count: a value is off by at most half of 2^-133, and an
+    fp32 sum of 96 products by half of 2^-149 each."""
+    rng = np.random.default_rng(5)
+    x = (rng.standard_normal((1, 20, 30, 96)) * (1.0 if small_weights else scale)).astype(np.float32)
+    wt = (rng.standard_normal((48, 96, 1, 1)) / 10 * (scale if small_weights else 1.0)).astype(np.float32)
+    out, kernel = _probe(x, wt, 1, (0, 0, 0, 0), None, 1, ACT_NONE)
+    assert kernel == "conv_split<64x32,1x1>"
+    ref = conv_ref(x.astype(np.float64), wt, None, (1, 1), (0, 0, 0, 0), ACT_NONE)
+    size = conv_ref(np.abs(x).astype(np.float64), np.abs(wt), None, (1, 1), (0, 0, 0, 0), ACT_NONE)
+    off = 2.0 ** -134 * (np.abs(x).sum(3)[..., None] if small_weights else np.abs(wt).sum((1, 2, 3)))
+    assert np.all(np.abs(out - ref) <= (96 / 16 + 8) * 2.0 ** -24 * size + off + 96 * 2.0 ** -149)
+
+
 @pytest.mark.parametrize("co,k", [(32, 32), (33, 20), (70, 100)])
 def test_packed_parts_are_the_weights(co, k):
     """The three parts of each weight add up to it within 2^-25, in the order
