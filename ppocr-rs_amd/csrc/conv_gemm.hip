@@ -2578,19 +2578,25 @@ static int pick_tile(int M, int cols, int dt) {
 }
 
 // The split kernel's tile for a layer, or -1 where the other kernels run it.
-// Measured against the fp32 kernels in the plans: 64x64 (128x32 up to 32
-// columns) from 512 tiles, two per CU, 1.0-1.3x, and from 256 where K is deep
-// enough to split (K >= 1024: the one-page medium detector's head and stem
-// 3x3 convs 1.29x and 1.24x).  Below that the 64x32 tile, whose waves halve
-// the serial work of a slice: 1.1-1.35x at K >= 256, 1.0-1.16x on the 40- to
-// 480-pixel layers of one line; its gated or K < 256 layers of more than 600
-// tiles 0.84-0.97x, so they stay.  128x128 tiles take K >= 768 layers that
-// leave at least 900 of them (three and a half rounds of two per CU):
-// 1.06-1.10x against 64x64 at K = 768-1024, 0.96-0.99x at K = 512; not the
-// gated layers, whose gate values would cost the second workgroup of a CU, nor
-// those of one image, which may leave SE channel sums from registers.  A
-// 96-column layer would leave a quarter of its 64-column tiles empty (the
-// batch-64 tiny recognizer's K = 192 ones 0.89-0.93x).
+// Measured against the fp32 kernels per layer, on the input of 42 detector
+// and recognizer plans (means of a class, fp32 time over split time): 64x64
+// (128x32 up to 32 columns) from 512 tiles, two per CU, 1.02-1.30x, and from
+// 256 where K is deep enough to split (K >= 1024: 1.08-1.32x).  Below that
+// the 64x32 tile, whose waves halve the serial work of a slice: 1.0x at up to
+// 64 tiles and K <= 128, else 1.02-1.34x (single layers 0.88-1.48x; the slow
+// ones are 3x3 layers of K = 576 and up to 150 tiles, 12-15 us each).  Its
+// layers of 600 tiles and more fill the GPU by themselves and gain only where
+// the products outweigh the split: 0.84-0.97x at K < 256, and from 850 tiles
+// 0.89-1.02x at K = 256 and, with an SE gate, whose values have to arrive as
+// well, 0.85-0.96x at K = 384 and 0.95-1.01x at K = 512 (gated at 600-700
+// tiles: 0.95-1.08x at K = 384, 1.08-1.11x at K = 512).  128x128 tiles take
+// K >= 768 layers that leave at least 900 of them (three and a half rounds of
+// two per CU): 1.06-1.10x against 64x64 at K = 768-1024, 0.96-0.99x at
+// K = 512; not the gated layers, whose gate values would cost the second
+// workgroup of a CU, nor those of one image, which may leave SE channel sums
+// from registers.  A 96-column layer would leave a quarter of its 64-column
+// tiles empty (the batch-64 tiny recognizer's K = 192 ones 0.89-0.93x).
+// Narrow layers of small K have no split weights (conv_takes_split3).
 static int split_tile(const ConvParams& p) {
   if (!p.wt3 || p.dt != DT_F32) return -1;
   const int M = p.N * p.Ho * p.Wo, K = p.kh * p.kw * p.C;
@@ -2599,7 +2605,7 @@ static int split_tile(const ConvParams& p) {
   };
   int t = p.Co <= 32 ? 2 : 0;
   if (tiles(t) < kSplitMinTiles && !(K >= 1024 && tiles(t) >= kSplitMinTiles / 2)) {
-    if (p.db_ch || (K < 256 && tiles(3) >= 600)) return -1;
+    if (p.db_ch || (tiles(3) >= 850 ? K <= (p.in_gate ? 512 : 256) : tiles(3) >= 600 && K < 256)) return -1;
     t = 3;
   } else if (t == 0 && p.Co <= 96 && p.Co % 64 != 0 && p.Co % 64 <= 32 && K < 256) {
     return -1;
@@ -2771,8 +2777,12 @@ static void launch_typed(const ConvParams& p, hipStream_t s) {
   }
 }
 
+// Layers of up to 64 columns need more K to outweigh the split of their input:
+// up to 32 columns 0.77-0.98x the fp32 kernels at K = 48 and 64 and 0.75-1.07x
+// at K = 96 (1.06-1.08x at K = 192), 64 columns 0.71-0.95x at K = 64 and up to
+// 1200 tiles (1.03-1.12x above).  Wider ones are even from K = 48 on.
 bool conv_takes_split3(int Co, int K) {
-  return Co >= 24 && K >= 48 && split3_size(Co, K) * 2 < kOutOfRange;
+  return Co >= 24 && K >= (Co <= 32 ? 128 : Co <= 64 ? 96 : 48) && split3_size(Co, K) * 2 < kOutOfRange;
 }
 
 bool conv_runs_split(const ConvParams& p) { return split_tile(p) >= 0; }

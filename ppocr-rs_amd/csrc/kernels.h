@@ -308,10 +308,11 @@ void launch_se_multi(const SeMulti& m, hipStream_t s);
 bool se_fused(const SeParams& p);
 
 // NCHW fp32 (3 planes) -> NHWC with 4 channels (fourth channel zero).
+void launch_nchw_to_nhwc4(const float* in, void* out, int N, int H, int W, int dt, hipStream_t s);
+
 // Copies bytes (a multiple of 4) between device and pinned host memory by a
 // kernel of the stream.
 void launch_host_copy(void* dst, const void* src, size_t bytes, hipStream_t s);
-void launch_nchw_to_nhwc4(const float* in, void* out, int N, int H, int W, int dt, hipStream_t s);
 
 // Max pool 2x2, stride 1, pads (0,0,1,1) into a channel slice.
 void launch_maxpool_same(const void* in, int N, int H, int W, int C, int in_ps, void* out, int out_ps, int dt,

@@ -35,3 +35,28 @@ def test_the_input_outlives_the_pass(kind, size, shape, bf16):
     """benchmark and profile replay a plan on an input that is uploaded once;
     an activation in its place would have the next replay run on that."""
     assert plan(kind, size, shape, bf16)[1]
+
+
+# Layers that the split kernel measured slower on than the fp32 kernels, and
+# neighbours of each in size, K or gate that it measured faster on.
+@pytest.mark.parametrize("kind,size,shape,layer,split", [
+    ("rec", "small", (6, 48, 500), "blocks.3.blocks.1.channel_conv1", False),  # gated K = 384, 864 64x32 tiles
+    ("det", "small", (8, 416, 736), "blocks.3.blocks.1.channel_conv1", False),  # gated K = 384, 912
+    ("det", "medium", (1, 416, 736), "blocks.2.blocks.1.channel_conv1", True),  # gated K = 512, 608
+    ("rec", "medium", (1, 48, 1200), "blocks.2.blocks.1.channel_conv1", False),  # gated K = 512, 928
+    ("rec", "medium", (1, 48, 320), "blocks.2.blocks.1.channel_conv1", True),  # gated K = 512, fewer
+    ("rec", "medium", (16, 48, 320), "blocks.0.blocks.0.channel_conv2", False),  # K = 256, 960
+    ("det", "small", (1, 160, 320), "blocks.1.blocks.1.channel_conv1", True),  # gated K = 96, 78
+    ("rec", "small", (64, 48, 320), "blocks.0.blocks.0.channel_conv1", True),  # gated K = 96, 64x64
+    ("det", "small", (8, 416, 736), "convolution.stem2b", False),  # K = 48, 24 columns
+    ("det", "small", (8, 416, 736), "input_conv.0.pointwise_convolution", False),  # K = 96, 24 columns
+    ("rec", "small", (64, 48, 320), "convolution.stem2a", True),  # K = 192, 24 columns
+    ("det", "medium", (4, 416, 736), "path_aggregation_lateral_convolution.0.pointwise", False),  # K = 64, 64 columns
+    ("det", "medium", (2, 416, 736), "convolution.stem4", True),  # K = 64, 128 columns
+    ("det", "medium", (8, 416, 736), "conv_up+conv_final", True),  # K = 64, 256 columns
+])
+def test_layers_run_on_the_faster_kernel(kind, size, shape, layer, split):
+    ops, _, _ = plan(kind, size, shape, greedy=kind == "rec")
+    kernels = [k for n, k in ops if n.endswith(layer)]
+    assert len(kernels) == 1
+    assert kernels[0].startswith("conv_split" if split else "conv_gemm"), kernels
