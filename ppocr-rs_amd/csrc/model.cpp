@@ -298,17 +298,15 @@ class Builder {
   struct Deferred {
     Op op;
     std::function<ConvParams(const Exec&)> fill;
-    ConvParams shape;  // its parameters with stand-in pointers
   };
 
   // With sp, the conv also leaves the channel sums of its output in *sp
   // where its kernel can (sp->P = 0 otherwise).  With `gated`, a bf16 layer
   // with an SE input gate returns there the x * g tensor its gate pass stores.
   // With `defer`, the op is returned there instead of added.
-  // `defer_split_k`: whether a deferred layer may split K (it then has its
-  // own launch).
+  // (Layers of a shared launch do not split K.)
   View conv(const View& x, const ConvW& w, const Epi& e, const std::string& name, SePartial* sp = nullptr,
-            View* gated = nullptr, Deferred* defer = nullptr, bool defer_split_k = true) {
+            View* gated = nullptr, Deferred* defer = nullptr) {
     if (x.c != w.ci_pad) raise(PPOCR_ERR_INVALID_MODEL, name + ": input has " + std::to_string(x.c) + " channels");
     const int Ho = (x.h + w.pt + w.pb - w.kh) / w.sh + 1;
     const int Wo = (x.w + w.pl + w.pr - w.kw) / w.sw + 1;
@@ -355,7 +353,7 @@ class Builder {
     base.dt = x.dt;
     size_t wo = w.w, bo = w.b, wo3 = w.w3;
     // Split-K workspace [splits][M][Co] fp32, live for this op only.
-    const int splits = defer && !defer_split_k ? 1 : conv_split_k(stand_in(base, a_src, w, has_ig && !prescale, 0));
+    const int splits = defer ? 1 : conv_split_k(stand_in(base, a_src, w, has_ig && !prescale, 0));
     View ws;
     if (splits > 1) ws = alloc(1, splits, x.n * Ho * Wo, w.co, name + ".split_k", DT_F32);
     base.splits = splits;
@@ -417,10 +415,7 @@ class Builder {
       launch_conv(fill(ex), s);
     };
     if (defer) {
-      ConvParams shape = stand_in(base, a_src, w, has_ig && !prescale, terms);
-      shape.splits = splits;
-      shape.se_part = has_part ? reinterpret_cast<float*>((uintptr_t)256) : nullptr;
-      *defer = Deferred{std::move(op), fill, shape};
+      *defer = Deferred{std::move(op), fill};
     } else {
       add_op(std::move(op));
     }
@@ -441,20 +436,22 @@ class Builder {
     return stand_in(p, x, w, false, 0);
   }
 
-  // Independent conv layers (the levels of a neck), each set of them that
-  // can share a launch (conv_multi_supported) as one op, the others one op
-  // each; a set is named after `name` with its first layer's index.
-  std::vector<View> conv_levels(const std::vector<const View*>& xs, const std::vector<ConvW>& ws, const Epi& e,
+  // Independent conv layers (the levels of a neck) with an epilogue of bias
+  // and activation, each set of them that can share a launch
+  // (conv_multi_supported) as one op, the others one op each; a set is named
+  // after `name` with its first layer's index.
+  std::vector<View> conv_levels(const std::vector<const View*>& xs, std::vector<ConvW> ws, int act,
                                 const std::vector<std::string>& names, const std::string& name,
                                 std::vector<SePartial>* sps = nullptr) {
     const int n = (int)xs.size();
-    std::vector<View> outs(n);
-    std::vector<Deferred> d(n);
+    Epi e;
+    e.act = act;
     // The levels run on one kind of kernel, the largest level's, so that they
-    // can share a launch: all on the split kernel, without splits of K (the
-    // small levels' workgroups fill in beside the large one's: the one-page
-    // medium detector's intraclass levels 78 launches for 90, 1.05x), or all
-    // on the fp32 kernels.
+    // can share a launch: all on the split kernel, where those of a set go
+    // without splits of K (the small levels' workgroups fill in beside the
+    // large one's: the one-page medium detector's intraclass levels 78 launches
+    // for 90, 1.05x), or all on the fp32 kernels.  A level with a launch of
+    // its own splits K as any layer does.
     bool split3 = true;
     size_t largest = 0;
     for (int i = 0; i < n; ++i) {
@@ -462,10 +459,14 @@ class Builder {
       if (xs[i]->pixels() > xs[largest]->pixels()) largest = i;
     }
     split3 = split3 && conv_runs_split(shape_of(*xs[largest], ws[largest]));
+    std::vector<ConvParams> shapes(n);
     for (int i = 0; i < n; ++i) {
-      ConvW w = ws[i];
-      if (!split3) w.w3 = NOW;
-      outs[i] = conv(*xs[i], w, e, names[i], sps ? &(*sps)[i] : nullptr, nullptr, &d[i], !split3);
+      if (!split3) ws[i].w3 = NOW;
+      ConvParams& p = shapes[i];
+      p = shape_of(*xs[i], ws[i]);
+      p.act = act;
+      p.splits = split3 ? 1 : conv_split_k(p);
+      if (sps && conv_se_blocks(p) > 0) p.se_part = reinterpret_cast<float*>((uintptr_t)256);
     }
     // Greedy sets in layer order: a layer joins the first set it can share a
     // launch with.
@@ -474,10 +475,10 @@ class Builder {
       bool placed = false;
       for (auto& set : sets) {
         if ((int)set.size() >= kConvMultiMax) continue;
-        std::vector<ConvParams> shapes;
-        for (int j : set) shapes.push_back(d[j].shape);
-        shapes.push_back(d[i].shape);
-        if (conv_multi_supported(shapes.data(), (int)shapes.size())) {
+        std::vector<ConvParams> trial;
+        for (int j : set) trial.push_back(shapes[j]);
+        trial.push_back(shapes[i]);
+        if (conv_multi_supported(trial.data(), (int)trial.size())) {
           set.push_back(i);
           placed = true;
           break;
@@ -485,26 +486,30 @@ class Builder {
       }
       if (!placed) sets.push_back({i});
     }
+    std::vector<View> outs(n);
     for (auto& set : sets) {
       if (set.size() == 1) {
-        add_op(std::move(d[set[0]].op));
+        const int i = set[0];
+        outs[i] = conv(*xs[i], ws[i], e, names[i], sps ? &(*sps)[i] : nullptr);
         continue;
       }
-      std::vector<Deferred*> members;
-      for (int j : set) members.push_back(&d[j]);
-      add_multi(members, sets.size() == 1 ? name : name + "." + std::to_string(set[0]));
+      std::vector<Deferred> d(set.size());
+      for (size_t k = 0; k < set.size(); ++k) {
+        const int i = set[k];
+        outs[i] = conv(*xs[i], ws[i], e, names[i], sps ? &(*sps)[i] : nullptr, nullptr, &d[k]);
+      }
+      add_multi(d, sets.size() == 1 ? name : name + "." + std::to_string(set[0]));
     }
     return outs;
   }
 
-  void add_multi(const std::vector<Deferred*>& d, const std::string& name) {
+  void add_multi(std::vector<Deferred>& d, const std::string& name) {
     Op op;
     op.name = name;
-    op.kernel = d[0]->op.kernel + "x" + std::to_string(d.size());
+    op.kernel = d[0].op.kernel + "x" + std::to_string(d.size());
     op.bound = 1;
     std::vector<std::function<ConvParams(const Exec&)>> fills;
-    for (Deferred* qp : d) {
-      Deferred& q = *qp;
+    for (Deferred& q : d) {
       op.flops += q.op.flops;
       op.bytes += q.op.bytes;
       op.reads.insert(op.reads.end(), q.op.reads.begin(), q.op.reads.end());
@@ -1307,7 +1312,7 @@ View rep_lk_fpn(Builder& B, const std::vector<View>& st, const int chans[4], int
     sws[i] = B.se_w(p + ".squeeze_excitation_block.conv1", p + ".squeeze_excitation_block.conv2", nc, nc / 4,
                     ACT_HSIG5);
   }
-  h = B.conv_levels(ins, iw, Epi{}, inames, "model.neck.insert_conv.in_conv", &sums);
+  h = B.conv_levels(ins, iw, ACT_NONE, inames, "model.neck.insert_conv.in_conv", &sums);
   // The four levels' gates (each from its conv's channel sums) in one launch.
   std::vector<View> g = B.se_levels(h, sws, "model.neck.insert_conv.se", sums);
   // fused[i] = h + h * g (+ up2(fused[i + 1])) feeds input_conv i's
@@ -1362,7 +1367,7 @@ View rep_lk_fpn(Builder& B, const std::vector<View>& st, const int chans[4], int
     reps[i] = 1 << i;
   }
   // The four pointwise convs in one launch where they share a kernel.
-  pt = B.conv_levels(pin, pws, Epi{}, pnames, "model.neck.input_conv.pointwise_convolution", &psums);
+  pt = B.conv_levels(pin, pws, ACT_NONE, pnames, "model.neck.input_conv.pointwise_convolution", &psums);
   // Every level's gate, then every level's x + x*g written upsampled into
   // its concat slot (deepest first in the channels): one launch each.
   std::vector<View> gi = B.se_levels(pt, psw, "model.neck.input_conv.se", psums);
@@ -1474,7 +1479,7 @@ std::vector<View> rank_one_levels(Builder& B, const std::vector<View>& xs, const
     pws[i] = r.pw;
     names[i] = p + ".pointwise";
   }
-  return B.conv_levels(dp, pws, Epi{}, names, prefix + ".pointwise");
+  return B.conv_levels(dp, pws, ACT_NONE, names, prefix + ".pointwise");
 }
 
 // fuse_intraclass_conv (src/cpu/model.rs:819-906).
@@ -1543,7 +1548,7 @@ View medium_neck(Builder& B, const std::vector<View>& st) {
       ws[i] = make_w(p);
       names[i] = p + suffix;
     }
-    return B.conv_levels(xp, ws, Epi{}, names, n + ".intraclass_blocks" + suffix);
+    return B.conv_levels(xp, ws, ACT_NONE, names, n + ".intraclass_blocks" + suffix);
   };
   std::vector<View> r = step(lat, [&](const std::string& p) {
     return B.conv_w(p + ".conv_reduce_channel", 64, 32, 1, 1, 1, 1, {0, 0, 0, 0}, true);

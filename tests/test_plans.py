@@ -60,3 +60,11 @@ def test_layers_run_on_the_faster_kernel(kind, size, shape, layer, split):
     kernels = [k for n, k in ops if n.endswith(layer)]
     assert len(kernels) == 1
     assert kernels[0].startswith("conv_split" if split else "conv_gemm"), kernels
+
+
+def test_a_level_with_its_own_launch_splits_k():
+    """The largest level of the medium neck's long step runs on wider tiles
+    than the others there: 299 of them, which K splits spread over the GPU."""
+    ops = dict(plan("det", "medium", (2, 416, 736))[0])
+    assert ops["model.neck.intraclass_blocks.0.long"] == "conv_split<128x32>+split_k3"
+    assert ops["model.neck.intraclass_blocks.long.1"] == "conv_split<64x32>x3"
