@@ -128,9 +128,11 @@ class Builder {
   }
 
   // OIHW [co][ci][kh][kw] -> [co][k = (ky*kw + kx)*ci_pad + c]; the padded
-  // input channels get zero weights.
+  // input channels get zero weights.  `as_conv`: a conv launch reads them, so
+  // fp32 plans also hold them split for the bf16 matrix cores; not the layers
+  // of the fused pair and linear kernels, which read the packed form.
   ConvW pack_conv(const std::vector<float>& W, const std::vector<float>& b, int ci, int co, int kh, int kw, int sh,
-                  int sw, std::vector<int> pads, int ci_pad = 0) {
+                  int sw, std::vector<int> pads, int ci_pad = 0, bool as_conv = true) {
     ConvW c;
     c.ci = ci;
     c.ci_pad = ci_pad ? ci_pad : ci;
@@ -147,7 +149,7 @@ class Builder {
           for (int kx = 0; kx < kw; ++kx)
             packed[(size_t)o * K + (size_t)(ky * kw + kx) * c.ci_pad + i] = W[(((size_t)o * ci + i) * kh + ky) * kw + kx];
     c.w = put_act(packed);
-    if (dt_ == DT_F32 && conv_takes_split3(co, (int)K)) {
+    if (dt_ == DT_F32 && as_conv && conv_takes_split3(co, (int)K)) {
       const size_t n = split3_size(co, (int)K);
       c.w3 = round_up(plan_.weights.size(), 256);
       plan_.weights.resize(c.w3 + n * 2);
@@ -187,14 +189,14 @@ class Builder {
 
   // Conv2d::load (src/cpu/model.rs:89-107) and Conv2d::load_bn (:110-131).
   ConvW conv_w(const std::string& p, int ci, int co, int kh, int kw, int sh, int sw, std::vector<int> pads, bool bias,
-               const std::string& norm = "", int ci_pad = 0) {
+               const std::string& norm = "", int ci_pad = 0, bool as_conv = true) {
     std::string wname = norm.empty() ? p + ".weight" : p + ".convolution.weight";
     std::string bname = norm.empty() ? p + ".bias" : p + ".convolution.bias";
     std::vector<float> W = get(wname, {co, ci, kh, kw}).v;
     std::vector<float> b;
     if (bias) b = get(bname, {co}).v;
     if (!norm.empty()) fold_bn(W, b, p + "." + norm, co);
-    return pack_conv(W, b, ci, co, kh, kw, sh, sw, pads, ci_pad);
+    return pack_conv(W, b, ci, co, kh, kw, sh, sw, pads, ci_pad, as_conv);
   }
 
   DwW dw_w(const std::string& p, int c, int kh, int kw, int sh, int sw, std::vector<int> pads, bool bias,
@@ -218,10 +220,10 @@ class Builder {
   }
 
   // Linear::new (src/cpu/backend.rs:1244-1280): weight [out][in] + bias.
-  ConvW linear_w(const std::string& p, int fin, int fout) {
+  ConvW linear_w(const std::string& p, int fin, int fout, bool as_conv = true) {
     std::vector<float> W = get(p + ".weight", {fout, fin}).v;
     std::vector<float> b = get(p + ".bias", {fout}).v;
-    return pack_conv(W, b, fin, fout, 1, 1, 1, 1, {0, 0, 0, 0});
+    return pack_conv(W, b, fin, fout, 1, 1, 1, 1, {0, 0, 0, 0}, 0, as_conv);
   }
 
   // ------------------------------------------------------------ values
@@ -1165,15 +1167,16 @@ View lcnet_block(Builder& B, const View& x, const std::string& p, BlockSpec s) {
   DwW tw = residual ? B.dw_w(p + ".token_conv", s.ci, 3, 3, s.sh, s.sw, {1, 1, 1, 1}, true)
                     : B.dw_w(p + ".token_conv", s.ci, 3, 3, s.sh, s.sw, {1, 1, 1, 1}, false, "normalization");
   bool has_se = s.se;
-  ConvW c1 = B.conv_w(p + ".channel_conv1", s.ci, 2 * s.ci, 1, 1, 1, 1, {0, 0, 0, 0}, false, "normalization");
-  ConvW c2 = B.conv_w(p + ".channel_conv2", 2 * s.ci, s.co, 1, 1, 1, 1, {0, 0, 0, 0}, false, "normalization");
+  const bool pays = pair_fusion_pays(x, s.ci, s.co, B.dt());
+  const std::vector<int> none = {0, 0, 0, 0};
+  ConvW c1 = B.conv_w(p + ".channel_conv1", s.ci, 2 * s.ci, 1, 1, 1, 1, none, false, "normalization", 0, !pays);
+  ConvW c2 = B.conv_w(p + ".channel_conv2", 2 * s.ci, s.co, 1, 1, 1, 1, none, false, "normalization", 0, !pays);
   // Without SE the token conv's output feeds only the pair: the pair
   // computes it per tile (src/cpu/backend.rs:697-816).
-  if (!has_se && pair_fusion_pays(x, s.ci, s.co, B.dt()))
+  if (!has_se && pays)
     return B.pointwise_pair(x, c1, c2, nullptr, residual, p + ".channel_conv", &tw);
   // A single image's fused pair forms the SE gate in its own prologue from
   // the token conv's channel sums (no gate launch) where the sums are few.
-  const bool pays = pair_fusion_pays(x, s.ci, s.co, B.dt());
   const bool fold = has_se && pays && x.n == 1;
   Builder::SePartial sums;
   View t = B.depthwise(x, tw, ACT_NONE, nullptr, p + ".token_conv", has_se ? s.ci / 4 : 0, &sums, nullptr, fold);
@@ -1768,7 +1771,7 @@ Plan build_recognizer(const SafeTensors& st, int size, const size_t nchw[4], int
       std::string p = e + ".svtr_block." + std::to_string(i);
       // fp32 plans fuse each block LayerNorm into the linear layer after it.
       const bool fuse_ln = ln_linear_supported(hid, 3 * hid, B.dt()) && ln_linear_supported(hid, mlp, B.dt());
-      ConvW qkv_w = B.linear_w(p + ".self_attn.qkv", hid, 3 * hid);
+      ConvW qkv_w = B.linear_w(p + ".self_attn.qkv", hid, 3 * hid, !fuse_ln);
       View qkv = fuse_ln ? B.ln_linear(h, p + ".layer_norm1", qkv_w, ACT_NONE, p + ".layer_norm1+qkv")
                          : B.conv(B.layer_norm(h, p + ".layer_norm1", nullptr, p + ".layer_norm1"), qkv_w, Epi{},
                                   p + ".self_attn.qkv");
@@ -1776,7 +1779,7 @@ Plan build_recognizer(const SafeTensors& st, int size, const size_t nchw[4], int
       Epi r1;
       r1.res = &h;
       View h1 = B.conv(ctx, B.linear_w(p + ".self_attn.projection", hid, hid), r1, p + ".self_attn.projection");
-      ConvW fc1_w = B.linear_w(p + ".mlp.fc1", hid, mlp);
+      ConvW fc1_w = B.linear_w(p + ".mlp.fc1", hid, mlp, !fuse_ln);
       View m = fuse_ln ? B.ln_linear(h1, p + ".layer_norm2", fc1_w, ACT_SILU, p + ".layer_norm2+fc1")
                        : B.conv(B.layer_norm(h1, p + ".layer_norm2", nullptr, p + ".layer_norm2"), fc1_w, silu,
                                 p + ".mlp.fc1");

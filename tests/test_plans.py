@@ -68,3 +68,10 @@ def test_a_level_with_its_own_launch_splits_k():
     ops = dict(plan("det", "medium", (2, 416, 736))[0])
     assert ops["model.neck.intraclass_blocks.0.long"] == "conv_split<128x32>+split_k3"
     assert ops["model.neck.intraclass_blocks.long.1"] == "conv_split<64x32>x3"
+
+
+@pytest.mark.parametrize("kind,size,limit", [("det", "tiny", 3.1e6), ("rec", "medium", 183.5e6)])
+def test_fused_layers_hold_no_split_weights(kind, size, limit):
+    """The pairs of the tiny detector and the layer-norm linear layers of the
+    medium recognizer read fp32 weights only (3.8 and 186.1 MB with both)."""
+    assert plan(kind, size, (1, 416, 736) if kind == "det" else (1, 48, 320))[2] < limit
