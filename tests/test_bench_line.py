@@ -90,3 +90,34 @@ def test_roof_follows_arithmetic_intensity():
     flops_rate = 6.4e9 / 0.05e-3
     attainable = 6.4e9 / 1.055e8 * bench.PEAK_HBM_GBS * 1e9
     assert abs(achieved / peak - flops_rate / attainable) < 1e-9
+
+
+def test_split_kernels_have_a_sixth_of_the_bf16_peak():
+    """An fp32 product as six bf16 ones: ridge 2500e12 / 6 / 8e12 = 52.1 FLOP/B
+    and a peak of 416.7 TFLOP/s for the kernels named conv_split, alone."""
+    bench = _bench()
+
+    def group(flops, nbytes):
+        return {"ms": 0.05, "flops": flops, "bytes": nbytes, "launches": 1, "bound": "mfma"}
+
+    above, below = group(5.3e9, 1e8), group(5.1e9, 1e8)  # 53 and 51 FLOP/B
+    assert bench.bound_of(above, "f32", "conv_split<64x64,1x1>") == "mfma"
+    assert bench.bound_of(below, "f32", "conv_split<64x32>x4") == "hbm"
+    assert bench.bound_of(below, "f32", "conv_gemm<64x32>") == "mfma"
+    achieved, peak, unit = bench.rate(above, "f32", "conv_split<64x64,1x1>")
+    assert (round(achieved, 6), round(peak, 3), unit) == (106.0, 416.667, "TFLOP/s")
+    assert bench.rate(below, "f32", "conv_split<64x64,1x1>") == (2000.0, 8000.0, "GB/s")
+
+
+def test_pass_rate_prices_each_kernel_at_its_roof():
+    """A pass at 300 TFLOP/s on split kernels is 0.72 of their roof, not 1.9
+    times the fp32 instructions'; a mixed one takes the sum of both times."""
+    bench = _bench()
+
+    def stat(kernel, flops):
+        return {"kernel": kernel, "bound": "mfma", "avg_ms": 1.0, "flops": flops, "bytes": 1e6}
+
+    split = [stat("conv_split<128x128,1x1>", 3e11)]
+    assert bench.pass_rates(split, 1.0, "f32")["frac_of_matrix_peak"] == 0.72
+    mixed = split + [stat("conv_gemm<64x64>", 1.573e10)]
+    assert bench.pass_rates(mixed, 1.0, "f32")["frac_of_matrix_peak"] == 0.82
