@@ -259,15 +259,16 @@ void check_input_len(ppocr_hip_model* m, const float* nchw, size_t len) {
           "input has " + std::to_string(len) + " values; the planned shape needs " + std::to_string(expected));
 }
 
-void check_input(ppocr_hip_model* m, const float* nchw, size_t len) {
-  check_input_len(m, nchw, len);
+// The finite check of an input.  Where the input's first chunk is already
+// queued it runs while the device computes, before anything is handed to the
+// caller.
+void check_finite(const float* nchw, size_t len) {
   if (!all_finite(nchw, len)) raise(PPOCR_ERR_INVALID_INPUT, "input contains non-finite values");
 }
 
-// The finite check of an input whose first chunk is already queued: it runs
-// while the device computes, before anything is handed to the caller.
-void check_queued_input(const float* nchw, size_t len) {
-  if (!all_finite(nchw, len)) raise(PPOCR_ERR_INVALID_INPUT, "input contains non-finite values");
+void check_input(ppocr_hip_model* m, const float* nchw, size_t len) {
+  check_input_len(m, nchw, len);
+  check_finite(nchw, len);
 }
 
 // Device pointer of the plan's NCHW staging buffer / output buffer.
@@ -321,9 +322,10 @@ void run_image_graph(ppocr_hip_model* m) {
   HIP_OK(hipGraphLaunch(m->image_graph ? m->image_graph : m->graph, m->ctx->stream));
 }
 
+bool output_fits(ppocr_hip_model* m, const float* out, size_t cap) { return out && cap >= output_elems(m); }
 void check_output_cap(ppocr_hip_model* m, const float* out, size_t cap) {
   const size_t n = output_elems(m);
-  if (!out || cap < n)
+  if (!output_fits(m, out, cap))
     raise(PPOCR_ERR_INVALID_INPUT, "output capacity " + std::to_string(cap) + " is below " + std::to_string(n));
 }
 
@@ -369,7 +371,7 @@ void run_batch(ppocr_hip_model* m, const float* nchw, size_t len, float* out) {
     upload_chunk(m, nchw, c);
     run_graph(m);
     if (c == 0) {
-      check_queued_input(nchw, len);
+      check_finite(nchw, len);
       populate_pages(out, output_elems(m) * sizeof(float));
     }
     download_chunk(m, out, c);
@@ -546,6 +548,7 @@ ppocr_status ppocr_hip_forward(ppocr_hip_model* model, const float* nchw, size_t
   return guarded([&] {
     if (!model) raise(PPOCR_ERR_INVALID_INPUT, "model is null");
     check_input_len(model, nchw, len);
+    if (!output_fits(model, out, out_cap)) check_finite(nchw, len);  // a bad input is refused before a bad output
     check_output_cap(model, out, out_cap);
     std::lock_guard<std::mutex> lock(model->ctx->mu);
     HIP_OK(hipSetDevice(model->ctx->device));
@@ -1297,6 +1300,7 @@ ppocr_status ppocr_hip_detect(ppocr_hip_model* model, const float* nchw, size_t 
     if (!model->plan.detector) raise(PPOCR_ERR_INVALID_INPUT, "detection needs a detector model");
     const ppocr_db_options o = db_options(options);
     check_input_len(model, nchw, len);
+    if (!transforms) check_finite(nchw, len);  // a bad input is refused first
     if (!transforms) raise(PPOCR_ERR_INVALID_INPUT, "transforms pointer is null");
     std::lock_guard<std::mutex> lock(model->ctx->mu);
     HIP_OK(hipSetDevice(model->ctx->device));
@@ -1308,7 +1312,7 @@ ppocr_status ppocr_hip_detect(ppocr_hip_model* model, const float* nchw, size_t 
     for (size_t c = 0; c < n_chunks(model); ++c) {
       upload_chunk(model, nchw, c);
       run_graph(model);
-      if (c == 0) check_queued_input(nchw, len);
+      if (c == 0) check_finite(nchw, len);
       const int items = (int)chunk_items(model, c);
       char* base = db_work(model->ctx, model->db_work, db_layout(items, (int)s[2], (int)s[3]).bytes);
       auto part = run_db(model->ctx, output_ptr(model), items, (int)s[2], (int)s[3], transforms + c * model->chunk, o,

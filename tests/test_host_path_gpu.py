@@ -8,6 +8,8 @@ queued and leaves the next call right; and calls of db_postprocess of growing
 and shrinking sizes, which share one buffer, agree with a fresh context.
 """
 
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -106,3 +108,33 @@ def test_maps_arrive_whole(gpu, n, h, w):
     got = gpu.db_postprocess(m, [(w, h, w, h)] * n)
     for g, v in zip(got, want):
         assert np.allclose(sorted(d.score for d in g), sorted(v), atol=1e-6)
+
+
+def test_a_bad_input_is_refused_first(gpu):
+    """A non-finite input is what is reported also where the output buffer is
+    too small or the transforms are missing."""
+    shape = (1, 3, 64, 96)
+    x = seeded.seeded_batch(1, 64, 96, 4)
+    det = ppocr_hip.Detector.load(gpu, model_path("det", "tiny"), "tiny", shape)
+    lib = ppocr_hip.lib()
+    out = np.empty(det.output_len, np.float32)
+    F = ctypes.POINTER(ctypes.c_float)
+
+    def forward(values, cap):
+        code = lib.ppocr_hip_forward(det.handle, values.ctypes.data_as(F), values.size, out.ctypes.data_as(F), cap)
+        return code, lib.ppocr_hip_last_error().decode() if code else ""
+
+    def detect(values):
+        counts, total = (ctypes.c_size_t * 1)(), ctypes.c_size_t()
+        code = lib.ppocr_hip_detect(det.handle, values.ctypes.data_as(F), values.size, None, None, None, 0, counts,
+                                    ctypes.byref(total))
+        return code, lib.ppocr_hip_last_error().decode() if code else ""
+
+    bad = x.copy()
+    bad.reshape(-1)[77] = np.nan
+    assert "capacity" in forward(x, out.size - 1)[1]
+    assert "non-finite" in forward(bad, out.size - 1)[1]
+    assert "transforms" in detect(x)[1]
+    assert "non-finite" in detect(bad)[1]
+    assert forward(x, out.size)[0] == 0
+    det.close()
