@@ -782,6 +782,166 @@ long ppocr_probe_plan_rounding(const char* path, int kind, int size, int n, int 
   }
 }
 
+// A 1x1 fp32 layer with its weights also split for the bf16 matrix cores and
+// the epilogue terms of a plan: x [n][h][w][c], weight [co][c], bias [co];
+// residual res [n][h][w][co] with res_gate [n][co] (both or the gate may be
+// null); up [n][h/up_s][w/up_s][co] (or null) added by nearest upsampling;
+// every output pixel written as a rep x rep block; out [n][h*rep][w*rep][co].
+// db_ch > 0: the DB head (co = 4 db_ch, act ReLU) with wf [db_ch][4] and bf,
+// out [n][4h][4w].  ctc: out [n*h*w][2], (class, probability) of each row.
+// *kernel: the instance that ran.  Returns 0, or 1 on a HIP error.
+int ppocr_probe_split_terms(const float* x, int n, int h, int w, int c, const float* weight, const float* bias, int co,
+                            int act, const float* res, const float* res_gate, const float* up, int up_s, int rep,
+                            int db_ch, const float* wf, float bf, int ctc, float* out, const char** kernel) {
+  static thread_local std::string name;
+  const size_t M = (size_t)n * h * w;
+  const size_t out_n = ctc ? 2 * M : db_ch ? 16 * M : M * rep * rep * co;
+  std::vector<void*> bufs;
+  bool ok = true;
+  auto room = [&](size_t bytes) {
+    void* d = nullptr;
+    ok = hipMalloc(&d, bytes) == hipSuccess && ok;
+    bufs.push_back(d);
+    return d;
+  };
+  auto put = [&](const float* src, size_t count) -> void* {
+    if (!src) return nullptr;
+    void* d = room(count * 4);
+    ok = ok && hipMemcpy(d, src, count * 4, hipMemcpyHostToDevice) == hipSuccess;
+    return d;
+  };
+  std::vector<uint16_t> parts(ppocr::split3_size(co, c));
+  ppocr::split3_weights(weight, co, c, parts.data());
+  ppocr::ConvParams p{};
+  p.in = put(x, M * c);
+  p.N = n, p.H = h, p.W = w, p.C = c, p.in_ps = c;
+  p.Ho = h, p.Wo = w, p.Co = co, p.out_ps = ctc ? 0 : db_ch ? 1 : co;
+  p.wt = put(weight, (size_t)co * c);
+  p.ldw = c;
+  void* wt3 = room(parts.size() * 2);
+  ok = ok && hipMemcpy(wt3, parts.data(), parts.size() * 2, hipMemcpyHostToDevice) == hipSuccess;
+  p.wt3 = wt3;
+  p.bias = static_cast<const float*>(put(bias, co));
+  p.kh = p.kw = p.sh = p.sw = 1;
+  p.act = act;
+  p.res = put(res, M * co);
+  p.res_ps = co;
+  p.res_gate = static_cast<const float*>(put(res_gate, (size_t)n * co));
+  p.up = put(up, up ? (size_t)n * (h / up_s) * (w / up_s) * co : 0);
+  p.up_s = up_s, p.up_ps = co;
+  p.rep = rep;
+  p.out_h = db_ch ? 4 * h : h * rep, p.out_w = db_ch ? 4 * w : w * rep;
+  p.dt = ppocr::DT_F32;
+  p.splits = 1;
+  p.db_ch = db_ch, p.db_bf = bf;
+  p.out_f32 = db_ch > 0;
+  p.db_wf = static_cast<const float*>(put(wf, (size_t)db_ch * 4));
+  void* d_out = room(out_n * 4);
+  int tiles = 0;
+  if (ctc) {
+    p.ctc_part = reinterpret_cast<float*>((uintptr_t)256);  // stands in where it chooses the tile
+    const int bn = ppocr::conv_tile_cols(p);
+    tiles = (co + bn - 1) / bn;
+    p.ctc_part = static_cast<float*>(room((size_t)3 * tiles * M * 4));
+  } else {
+    p.out = d_out;
+  }
+  name = ppocr::conv_kernel_name(p);
+  *kernel = name.c_str();
+  if (db_ch && ppocr::conv_tile_cols(p) % db_ch) ok = false;
+  if (up && (h % up_s || w % up_s)) ok = false;
+  if (ok) {
+    ppocr::launch_conv(p, nullptr);
+    if (ctc) ppocr::launch_ctc_merge(p.ctc_part, (int)M, tiles, static_cast<float*>(d_out), nullptr);
+    ok = hipGetLastError() == hipSuccess && hipDeviceSynchronize() == hipSuccess &&
+         hipMemcpy(out, d_out, out_n * 4, hipMemcpyDeviceToHost) == hipSuccess;
+  }
+  for (void* d : bufs)
+    if (d) (void)hipFree(d);
+  return ok ? 0 : 1;
+}
+
+// Up to kConvMultiMax k x k fp32 layers (stride 1, padding k / 2) with split
+// weights, as one launch and one by one: dims [count][n h w c co k], the
+// layers' x, weight [co][c][k][k] and bias one after the other; outputs
+// [n][h][w][co] likewise into `multi` and `single`; with se_multi and
+// se_single (one image, 1x1) also the SE channel sums, conv_se_blocks() rows of
+// co per layer.  *kernel: the first layer's instance.  Returns 0, 1 on a HIP
+// error, or 2 if the layers cannot share a launch.
+int ppocr_probe_split_multi(int count, const int* dims, const float* x, const float* weight, const float* bias, int act,
+                            float* multi, float* single, float* se_multi, float* se_single, const char** kernel) {
+  static thread_local std::string name;
+  std::vector<void*> bufs;
+  bool ok = true;
+  auto room = [&](size_t bytes) {
+    void* d = nullptr;
+    ok = hipMalloc(&d, bytes) == hipSuccess && ok;
+    bufs.push_back(d);
+    return d;
+  };
+  auto put = [&](const void* src, size_t bytes) {
+    void* d = room(bytes);
+    ok = ok && hipMemcpy(d, src, bytes, hipMemcpyHostToDevice) == hipSuccess;
+    return d;
+  };
+  ppocr::ConvMulti m{};
+  m.count = count;
+  std::vector<size_t> outs(count), sums(count, 0);
+  for (int i = 0; i < count; ++i) {
+    const int *d = dims + 6 * i, n = d[0], h = d[1], w = d[2], c = d[3], co = d[4], k = d[5];
+    const int K = k * k * c;
+    std::vector<float> packed((size_t)co * K);
+    for (int o = 0; o < co; ++o)
+      for (int ci = 0; ci < c; ++ci)
+        for (int t = 0; t < k * k; ++t)
+          packed[(size_t)o * K + (size_t)t * c + ci] = weight[((size_t)o * c + ci) * k * k + t];
+    std::vector<uint16_t> parts(ppocr::split3_size(co, K));
+    ppocr::split3_weights(packed.data(), co, K, parts.data());
+    ppocr::ConvParams& p = m.p[i];
+    p.in = put(x, (size_t)n * h * w * c * 4);
+    p.N = n, p.H = h, p.W = w, p.C = c, p.in_ps = c;
+    p.Ho = h, p.Wo = w, p.Co = co, p.out_ps = co;
+    p.wt = put(packed.data(), packed.size() * 4);
+    p.ldw = K;
+    p.wt3 = put(parts.data(), parts.size() * 2);
+    p.bias = static_cast<const float*>(put(bias, (size_t)co * 4));
+    p.kh = p.kw = k, p.sh = p.sw = 1, p.pt = p.pl = k / 2;
+    p.act = act;
+    p.up_s = 2, p.rep = 1, p.out_h = h, p.out_w = w;
+    p.dt = ppocr::DT_F32;
+    p.splits = 1;
+    outs[i] = (size_t)n * h * w * co;
+    p.out = room(outs[i] * 4);
+    if (se_multi) {
+      sums[i] = (size_t)ppocr::conv_se_blocks(p) * co;
+      if (sums[i]) p.se_part = static_cast<float*>(room(sums[i] * 4));
+    }
+    x += (size_t)n * h * w * c, weight += (size_t)co * K, bias += co;
+  }
+  int rc = 0;
+  if (ok && !ppocr::conv_multi_supported(m.p, count)) rc = 2;
+  name = ppocr::conv_kernel_name(m.p[0]);
+  *kernel = name.c_str();
+  for (int pass = 0; pass < 2 && ok && rc == 0; ++pass) {
+    for (int i = 0; i < count && ok; ++i) ok = hipMemset(m.p[i].out, 0xff, outs[i] * 4) == hipSuccess;
+    if (pass == 0)
+      ppocr::launch_conv_multi(m, nullptr);
+    else
+      for (int i = 0; i < count; ++i) ppocr::launch_conv(m.p[i], nullptr);
+    ok = ok && hipGetLastError() == hipSuccess && hipDeviceSynchronize() == hipSuccess;
+    float *o = pass == 0 ? multi : single, *s = pass == 0 ? se_multi : se_single;
+    for (int i = 0; i < count && ok; ++i) {
+      ok = hipMemcpy(o, m.p[i].out, outs[i] * 4, hipMemcpyDeviceToHost) == hipSuccess;
+      if (sums[i]) ok = hipMemcpy(s, m.p[i].se_part, sums[i] * 4, hipMemcpyDeviceToHost) == hipSuccess && ok;
+      o += outs[i];
+      if (s) s += sums[i];
+    }
+  }
+  for (void* d : bufs)
+    if (d) (void)hipFree(d);
+  return ok ? rc : 1;
+}
+
 // A model's plan, built on the host from a safetensors file (no device work),
 // as lines "<op>\t<kernel>", then "input kept" unless another buffer shares
 // arena bytes with the input, and "weights <bytes>".  Arguments and result as
