@@ -1392,11 +1392,15 @@ __global__ __launch_bounds__(256) void conv_gemm_direct_multi_kernel(ConvMulti m
 // off by up to half of that.
 //
 // What bounds it: six 32x32x16 MFMAs do the work of eight times as many fp32
-// ones' cycles (2.5 / 6 = 0.42 PFLOP/s against 0.157), and on dense random
-// operands the chip holds about half of that: 165-190 TFLOP/s on the
-// recognizer's K = 512-1024 layers (bf16 MFMA rate 1.0-1.14 PFLOP/s; the
-// library's bf16 product of 8192^3 reaches 1.23), where the fp32 kernel
-// above reaches 120-128.
+// ones' cycles (2.5 / 6 = 0.42 PFLOP/s against 0.157).  Of that the 64x64 tile
+// reaches 100-150 and the 128x128 tile 180 TFLOP/s on the recognizer's K =
+// 512-1024 layers, where the fp32 kernel above reaches 120-128.  Counters
+// there: the clock is 1.9 of 2.4 GHz under the load (2.4-2.5 beside it); at
+// that clock the 64x64 tile's vector pipes are 68 % busy (75 % gated), since
+// both column waves split every A fragment, and its matrix pipes 42 %, the
+// 128x128 tile's 39 % and 53 %; LDS accesses take 12-17 % of the cycles, and
+// waves wait 27-34 % of theirs.  On the detector's smaller maps 49-62 % and
+// 24-38 % at 2.0-2.3 GHz.
 //
 // Layout: the weights are split and put in MFMA operand order at load
 // (split3_weights): 1 KB per 32 columns, 16 k values and part, so a wave's

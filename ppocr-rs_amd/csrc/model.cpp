@@ -451,9 +451,10 @@ class Builder {
     // The levels run on one kind of kernel, the largest level's, so that they
     // can share a launch: all on the split kernel, where those of a set go
     // without splits of K (the small levels' workgroups fill in beside the
-    // large one's: the one-page medium detector's intraclass levels 78 launches
-    // for 90, 1.05x), or all on the fp32 kernels.  A level with a launch of
-    // its own splits K as any layer does.
+    // large one's: the medium detector's intraclass 7x7, 5x5 and 3x3 steps take
+    // 0.3-0.8 of the separate fp32 launches' time at one to eight pages, one
+    // page 78 launches for 90), or all on the fp32 kernels.  A level with a
+    // launch of its own splits K as any layer does.
     bool split3 = true;
     size_t largest = 0;
     for (int i = 0; i < n; ++i) {
